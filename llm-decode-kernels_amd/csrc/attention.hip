@@ -52,9 +52,11 @@
 // they weight V, the V sum and the normalisation in fp32, the output rounded once to fp16.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "attention.h"
 #include "ldk_common.h"
+#include "lds_dma.h"
 #include "warm.h"
 
 namespace {
@@ -493,7 +495,7 @@ __global__ __launch_bounds__(64) void attention_merge_kernel(const int64_t* pos_
 // ------------------------------------------------------------ prompt (many-token) attention
 //
 // ldk_prefill_attention: T tokens of one sequence at positions pos[T], in two launches.
-//  1. prefill_rope_kv_kernel, one workgroup per token: the decode kernel's fp16 RoPE (same cos and
+//  1. prefill_rope_kv_kernel, 16 tokens per workgroup: the decode kernel's fp16 RoPE (same cos and
 //     sin of pos * inv_freq, same roundings) on the token's q heads, written to q_scratch
 //     [T][nq][128], and on its k heads, written with its v heads into the tiled caches at pos[t]
 //     (a position outside [0, max_len) writes nothing).
@@ -507,38 +509,95 @@ __global__ __launch_bounds__(64) void attention_merge_kernel(const int64_t* pos_
 // The launch boundary orders the cache writes of launch 1 before the reads of launch 2.
 constexpr int kPWaves = 4;
 
-__global__ __launch_bounds__(256) void prefill_rope_kv_kernel(const half_t* qkv, int64_t ldqkv, const int64_t* pos,
+// A workgroup takes 16 tokens and every gridDim.y-th of their nq + 2 nkv heads; thread (tok, p) has
+// dims 4p .. 4p + 3 and 64 above of one token (8 p .. 8p + 7 of a v head). The 16 x 64 angles' fp16
+// cos and sin are formed once, through LDS. V^T rows run along positions, so a v head is turned in
+// LDS and stored with the tokens along the lanes (32 contiguous bytes per dim where the positions
+// are consecutive) instead of one 2-byte store to its own line per element. One workgroup per token
+// with 2-byte accesses took 10.7 us at 3000 tokens of 12/2 heads and 16.3 at 816 of 16/16; this takes
+// 7.6 and 8.0. VEC: 8- and 16-byte accesses to qkv (its base and row stride allow them).
+constexpr int kRopeTok = 16;
+
+template <bool VEC>
+__global__ __launch_bounds__(256) void prefill_rope_kv_kernel(const half_t* qkv, int64_t ldqkv, const int64_t* pos, int T,
                                                               const float* inv_freq, half_t* kc, half_t* vt,
                                                               half_t* qs, int nq, int nkv, int L) {
-  // every element a thread ropes has dim pair j = tid % 64 (the loops step by 256), so each thread
-  // forms its own cos and sin: no shared table and no barrier, and the row loads need not wait
-  // for the position
-  const int t = blockIdx.x, tid = threadIdx.x, jt = tid & 63;
-  const int64_t p = pos[t];
-  const float ang = (float)p * inv_freq[jt];
-  const half_t cj = (half_t)cosf(ang), sj = (half_t)sinf(ang);
+  __shared__ __align__(16) half_t cs[2][kRopeTok][64];
+  __shared__ __align__(16) half_t vs[kRopeTok][kHD + 2];
+  const int tid = threadIdx.x, t0 = (int)blockIdx.x * kRopeTok;
+  const int tok = tid >> 4, p = tid & 15;
+  const int t = min(t0 + tok, T - 1);  // tokens past T repeat the last one; they store nothing
+  const bool in = t0 + tok < T;
+  auto load = [&](const half_t* src, auto& v) __attribute__((always_inline)) {
+    using V = std::remove_reference_t<decltype(v)>;
+    if constexpr (VEC) {
+      v = *reinterpret_cast<const V*>(src);
+    } else {
+#pragma unroll
+      for (int e = 0; e < (int)(sizeof(V) / 2); ++e) v[e] = src[e];
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < kRopeTok * 64 / 256; ++i) {
+    const int a = tid + 256 * i, at = a >> 6, j = a & 63;
+    const float ang = (float)pos[min(t0 + at, T - 1)] * inv_freq[j];
+    cs[0][at][j] = (half_t)cosf(ang);
+    cs[1][at][j] = (half_t)sinf(ang);
+  }
+  const int64_t pi = pos[t];
+  const bool wr = in && pi >= 0 && pi < L;
+  const int pp = wr ? (int)pi : 0;
+  // the v store's element: token tid % 16, dims tid / 16 + 16 i
+  const int64_t pv = pos[min(t0 + (tid & 15), T - 1)];
+  const bool wv = t0 + (tid & 15) < T && pv >= 0 && pv < L;
   const half_t* row = qkv + (int64_t)t * ldqkv;
-  half_t* qo = qs + (int64_t)t * nq * kHD;
-  for (int e = tid; e < nq * 64; e += 256) {  // (head, dim pair j < 64): dims j and j + 64
-    const int h = e >> 6, j = e & 63;
-    half_t x0 = row[h * kHD + j], x1 = row[h * kHD + j + 64];
-    rope_rotate(x0, x1, cj, sj);
-    qo[h * kHD + j] = x0;
-    qo[h * kHD + j + 64] = x1;
+  __syncthreads();
+  half4_t c, sn;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    c[e] = cs[0][tok][4 * p + e];
+    sn[e] = cs[1][tok][4 * p + e];
   }
-  if (p < 0 || p >= L) return;  // uniform
-  const int pp = (int)p;
-  for (int e = tid; e < nkv * 64; e += 256) {
-    const int h = e >> 6, j = e & 63;
-    half_t x0 = row[(nq + h) * kHD + j], x1 = row[(nq + h) * kHD + j + 64];
-    rope_rotate(x0, x1, cj, sj);
-    half_t* kw = kc + (int64_t)h * L * kHD;
-    kw[k_offset(pp, j)] = x0;
-    kw[k_offset(pp, j + 64)] = x1;
-  }
-  for (int e = tid; e < nkv * kHD; e += 256) {
-    const int h = e >> 7, d = e & (kHD - 1);
-    vt[(int64_t)h * kHD * L + vt_offset(d, pp)] = row[(nq + nkv + h) * kHD + d];
+  for (int h = (int)blockIdx.y; h < nq + 2 * nkv; h += (int)gridDim.y) {
+    if (h < nq + nkv) {  // uniform
+      half4_t x0, x1;
+      load(row + (int64_t)h * kHD + 4 * p, x0);
+      load(row + (int64_t)h * kHD + 64 + 4 * p, x1);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        half_t a = x0[e], b = x1[e];
+        rope_rotate(a, b, c[e], sn[e]);
+        x0[e] = a;
+        x1[e] = b;
+      }
+      if (h < nq) {
+        if (in) {
+          half_t* qo = qs + ((int64_t)t * nq + h) * kHD;
+          *reinterpret_cast<half4_t*>(qo + 4 * p) = x0;
+          *reinterpret_cast<half4_t*>(qo + 64 + 4 * p) = x1;
+        }
+      } else if (wr) {
+        half_t* kw = kc + (int64_t)(h - nq) * L * kHD;
+        *reinterpret_cast<half4_t*>(kw + k_offset(pp, 4 * p)) = x0;
+        *reinterpret_cast<half4_t*>(kw + k_offset(pp, 64 + 4 * p)) = x1;
+      }
+    } else {
+      half8_t v;
+      load(row + (int64_t)h * kHD + 8 * p, v);
+      __syncthreads();  // the v head before has been read
+#pragma unroll
+      for (int e = 0; e < 8; e += 2)
+        *reinterpret_cast<half2_t*>(&vs[tok][8 * p + e]) = half2_t{v[e], v[e + 1]};
+      __syncthreads();
+      if (wv) {
+        half_t* vw = vt + (int64_t)(h - nq - nkv) * kHD * L;
+#pragma unroll
+        for (int i = 0; i < kHD / 16; ++i) {
+          const int d = (tid >> 4) + 16 * i;
+          vw[vt_offset(d, (int)pv)] = vs[tid & 15][d];
+        }
+      }
+    }
   }
 }
 
@@ -681,6 +740,296 @@ __global__ __launch_bounds__(kPWaves * 64) void prefill_attention_kernel(const h
       acc = __builtin_fmaf(ov[w], f, acc);
     }
     out[(int64_t)(t0 + j) * ldo + (int64_t)h * kHD + d] = (half_t)(l > 0.0f ? acc / l : 0.0f);
+  }
+}
+
+// ---- the same attention for blocks of tokens that share K and V through LDS
+//
+// prefill_attention_kernel reads 16 KB of K and V from L2 into registers for every 32 positions x
+// 16 tokens, which bounds it (about 190 TFLOP/s, 12 TB/s from the L2s, at 3000 tokens of 12/2
+// heads). Here a workgroup of CG x KG waves takes 32 CG tokens of one query head: wave (kg, cg)
+// has 32 tokens (two MFMA column tiles) over the 32-position steps kg, kg + KG, ... The waves of a
+// K group share each step's K and V tiles through an S-slot LDS ring filled by 16-byte loads to
+// LDS (a tile's lane l reads the 16 bytes lane l wrote: no bank conflicts), so a byte from L2
+// serves 32 CG tokens and a byte from LDS 32.
+//
+// One barrier per step; a step's V (and with four slots the next step's K) leaves LDS before the
+// MFMAs ahead of the ones that need it. P.V is O^T = V^T P with the token as the column, so a
+// lane's score, maximum, sum and output columns are the same token and the online softmax needs
+// no shuffles beyond the reduction over a tile's rows. Steps in which no token of the block masks
+// a position run without masks. The K groups' (m, l, O) meet in LDS at the end.
+//
+// Per token numerics are prefill_attention_kernel's: its mask, its clearing of V past each
+// 16-token tile's last position, fp16 numerators, fp32 sums; the softmax scale is applied in the
+// exponent, exp2((s - m) * scale * log2 e), with one fma instead of a product and a difference.
+//
+// What bounds it: about 4 vector instructions per MFMA (exponent, sum, conversion, maximum), which
+// take the wave's issue slots next to the MFMAs' (one MFMA with four fma's between takes 24 cycles
+// on this chip, 16 without), and 32 KB of loads to LDS per 32 positions of a workgroup. Measured
+// (both launches, graph replays, us): 12/2 heads at 3000 tokens 148 -> 71, at 6000 463 -> 172, 1024
+// after 3000 cached 104 -> 61; 28/4 heads at 1500 105 -> 49; 16/16 at 816 44 -> 29 (of these the
+// first launch 10.7 -> 7.6 and 16.3 -> 8.0).
+constexpr int kStepBytes = 2 * kChunk * kHD * 2;  // K and V of one step
+
+template <int CG, int KG, int S>
+__global__ __launch_bounds__(CG* KG * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attention_block_kernel(const half_t* qs, const int64_t* pos, int T,
+                                                                     const half_t* kc, const half_t* vt, half_t* out,
+                                                                     int64_t ldo, int nq, int nkv, int L,
+                                                                     float scale) {
+  constexpr int BT = 32 * CG;             // tokens per workgroup
+  constexpr int KB = kStepBytes / 2;      // bytes of a step's K (and of its V): 8 tiles
+  constexpr int LI = 8 / CG;              // K (and V) tiles each wave loads per step
+  constexpr bool AHEAD = S >= 4;          // deep enough to read the next step's K a step early
+  static_assert(CG * LI == 8 && S >= 2, "whole loads per wave, two slots");
+  __shared__ __align__(16) unsigned char ring[KG * S * kStepBytes];
+  __shared__ float mls[CG * KG][4][64];  // the K groups' m and l per column tile and lane
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave / CG, cg = wave % CG;
+  const int c16 = lane & 15, kb = lane >> 4;
+  const int h = (int)blockIdx.x, t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * BT;  // longest blocks first
+  const int kvh = __builtin_amdgcn_readfirstlane(h / (nq / nkv));
+  const int nt = min(BT, T - t0);
+
+  // the first and last of the positions that the block's tokens attend up to, and so the steps in
+  // which no score is masked and all of its steps
+  int pb = -1, pa = kMaxLen;
+#pragma unroll
+  for (int i = 0; i < BT; i += 64)
+    if (i + lane < nt) {
+      const int64_t pp = pos[t0 + i + lane];
+      const int p = pp < 0 ? -1 : pp >= L ? L - 1 : (int)pp;
+      pb = max(pb, p);
+      pa = min(pa, p);
+    }
+  const int pblk = __builtin_amdgcn_readfirstlane((int)wave_max((float)pb));  // exact: below 2^24
+  const int pfull = __builtin_amdgcn_readfirstlane(-(int)wave_max((float)-pa));
+  const int nsteps = pblk < 0 ? 0 : pblk / kChunk + 1;
+  const int n = (nsteps + KG - 1) / KG;   // steps of a K group (the last ones may be dead)
+  const int nfull = (pfull + 1) / kChunk / KG;  // of them, steps that no token masks
+
+  // this wave's columns: token t0 + 32 cg + 16 ct + c16 and its last position (columns past T are
+  // not masked and not stored); the last position of each column tile
+  int plim[2], pmax[2];
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct) {
+    const int col = 32 * cg + 16 * ct + c16;
+    int pl = -1;
+    if (col < nt) {
+      const int64_t pp = pos[t0 + col];
+      pl = pp < 0 ? -1 : pp >= L ? L - 1 : (int)pp;
+    }
+    pmax[ct] = __builtin_amdgcn_readfirstlane((int)wave_max((float)pl));
+    plim[ct] = col < nt ? pl : kMaxLen;
+  }
+  const int plast = max(pmax[0], pmax[1]);  // the wave's last position: later steps hold nothing for it
+
+  // K or V of step j of this K group into slot j % S (steps past the block's load nothing)
+  const u32x4 krs = ldk::raw_rsrc_uniform(kc + (int64_t)kvh * L * kHD, (uint32_t)L * kHD * 2);
+  const u32x4 vrs = ldk::raw_rsrc_uniform(vt + (int64_t)kvh * kHD * L, (uint32_t)L * kHD * 2);
+  const uint32_t lane_off = (uint32_t)(c16 * 64 + kb * 16);
+  unsigned char* const kring = ring + kg * S * kStepBytes;
+  unsigned char* const vring = kring + KB;
+  auto load = [&](u32x4 rs, unsigned char* slots, int j) __attribute__((always_inline)) {
+    const int st = j * KG + kg;
+    const uint32_t off = st < nsteps ? (uint32_t)st * KB + lane_off : kDead;
+#pragma unroll
+    for (int i = 0; i < LI; ++i)
+      ldk::dma_buffer16(rs, off + (uint32_t)((cg * LI + i) * 1024), 0u,
+                        ldk::lds_addr(slots + (j % S) * kStepBytes + (cg * LI + i) * 1024));
+  };
+#pragma unroll
+  for (int j = 0; j < S - 1; ++j) {
+    load(krs, kring, j);
+    load(vrs, vring, j);
+  }
+
+  // this wave's q operands: waited for here, once, so that the compiler has no load of its own
+  // left to wait for inside the loop (its count does not know the loads to LDS)
+  u32x4 q[2][4];
+  {
+    const auto qrs = ldk::buffer_rsrc(qs, (uint32_t)((int64_t)T * nq * kHD * 2));
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct) {
+      const int col = 32 * cg + 16 * ct + c16;
+      uint32_t dq = col < nt ? 0u : kDead;
+      asm volatile("" : "+v"(dq));
+      const uint32_t oq = (uint32_t)(((int64_t)(t0 + col) * nq + h) * kHD * 2) | dq;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) q[ct][s] = ldk::buffer_load16(qrs, oq + (uint32_t)((8 * kb + 32 * s) * 2));
+    }
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) asm volatile("" : "+v"(q[ct][s]));
+  }
+
+  const float sc = scale * 1.44269504088896341f;
+  float m_run[2] = {-__builtin_inff(), -__builtin_inff()}, l_lane[2] = {0.0f, 0.0f};
+  float4_t o[2][8];        // O^T[dim 16b + 4kb + r][token c16], unnormalised
+  float4_t acc[2][2];      // [row half hb][column tile]: scores of positions 8kb + 4hb + r
+  u32x4 ph[2];             // numerators, fp16: the B operand of P.V
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+    for (int b = 0; b < 8; ++b) o[ct][b] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+  // the 8 tiles of a step's K or V, read ahead of the MFMAs before the ones that use them
+  u32x4 kt[8], vv[8];
+  auto tiles = [&](u32x4 (&t)[8], const unsigned char* src) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t[i] = *reinterpret_cast<const u32x4*>(src + i * 1024 + lane * 16);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto scores = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct) acc[hb][ct] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) acc[hb][ct] = mfma16(kt[4 * hb + s], q[ct][s], acc[hb][ct]);
+  };
+  auto pv = [&](auto maskedc, int cb0) __attribute__((always_inline)) {
+    uint32_t mk[2][4];
+    if constexpr (decltype(maskedc)::value) {  // zero V past the tile's last position (0 x NaN)
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct) {
+        const int last = pmax[ct] - cb0 - 8 * kb;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          mk[ct][e] = (2 * e <= last ? 0x0000FFFFu : 0u) | (2 * e + 1 <= last ? 0xFFFF0000u : 0u);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct) {
+        u32x4 v = vv[b];
+        if constexpr (decltype(maskedc)::value)
+          v = u32x4{v[0] & mk[ct][0], v[1] & mk[ct][1], v[2] & mk[ct][2], v[3] & mk[ct][3]};
+        o[ct][b] = mfma16(v, ph[ct], o[ct][b]);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // The rescale is skipped while no token of the tile sees a larger score (its factor is then 1 in
+  // every lane). Letting the maximum lag by up to 2^8 would skip it in nearly every step (12/2 heads
+  // at 3000 tokens 64 instead of 71 us), but the largest numerators are then rounded instead of
+  // exactly 1: 1.7% more error against 64 bits.
+  float base[2] = {0.0f, 0.0f};  // m_run * sc, 0 while m_run is -inf
+  auto softmax = [&](auto maskedc, int cb0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct) {
+      float mc = -__builtin_inff();
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if constexpr (decltype(maskedc)::value)
+          if (cb0 + 8 * kb + e > plim[ct]) acc[e >> 2][ct][e & 3] = -__builtin_inff();
+        mc = fmaxf(mc, acc[e >> 2][ct][e & 3]);
+      }
+      mc = max_xor32(max_xor16(mc));
+      if (__any(mc > m_run[ct])) {
+        const float m_new = fmaxf(m_run[ct], mc);
+        // a token with no live position so far keeps m = -inf; its factor is taken against 0
+        const float alpha = __builtin_amdgcn_exp2f((m_run[ct] - (m_new == -__builtin_inff() ? 0.0f : m_new)) * sc);
+        l_lane[ct] *= alpha;
+#pragma unroll
+        for (int b = 0; b < 8; ++b) o[ct][b] *= alpha;
+        m_run[ct] = m_new;
+        base[ct] = m_new == -__builtin_inff() ? 0.0f : m_new * sc;
+      }
+      half8_t p;
+      float ls = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[e >> 2][ct][e & 3], sc, -base[ct]));
+        ls += x;
+        p[e] = (half_t)x;
+      }
+      ph[ct] = __builtin_bit_cast(u32x4, p);
+      l_lane[ct] += ls;
+    }
+  };
+  auto step = [&](auto maskedc, int j) __attribute__((always_inline)) {
+    // stage j (and with a deep ring j + 1) has landed, and every wave is done with step j - 1,
+    // whose slot takes stage j + S - 1
+    ldk::wait_vm<AHEAD ? (S - 3) * 2 * LI : (S - 2) * 2 * LI>();
+    ldk::ring_barrier();
+    const int cb0 = (j * KG + kg) * kChunk;
+    const bool live = !decltype(maskedc)::value || cb0 <= plast;  // uniform
+    if (!AHEAD && live) tiles(kt, kring + (j % S) * kStepBytes);
+    if (live) {
+      tiles(vv, vring + (j % S) * kStepBytes);
+      scores();
+    }
+    load(krs, kring, j + S - 1);
+    if (AHEAD) tiles(kt, kring + ((j + 1) % S) * kStepBytes);
+    if (live) softmax(maskedc, cb0);
+    load(vrs, vring, j + S - 1);
+    if (live) pv(maskedc, cb0);
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0): no LDS read is left pending
+  };
+  ldk::wait_vm<0>();  // the first stages, with q
+  ldk::ring_barrier();
+  if (AHEAD) tiles(kt, kring);
+  for (int j = 0; j < nfull; ++j) step(IntC<0>(), j);
+  for (int j = nfull; j < n; ++j) step(IntC<1>(), j);
+  ldk::wait_vm<0>();
+  __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+  ldk::ring_barrier();  // the ring is free: every wave's loads have landed and its reads are done
+
+  // ---- the K groups meet: groups past the first leave m, l and O, lane for lane
+  float l_w[2];
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct) l_w[ct] = ldk::add_xor32(ldk::add_xor16(l_lane[ct]));
+  float4_t* const red = reinterpret_cast<float4_t*>(ring);  // [wave - CG][16][64]
+  if (kg > 0) {
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct) {
+      mls[wave][2 * ct][lane] = m_run[ct];
+      mls[wave][2 * ct + 1][lane] = l_w[ct];
+#pragma unroll
+      for (int b = 0; b < 8; ++b) red[((wave - CG) * 16 + 8 * ct + b) * 64 + lane] = o[ct][b];
+    }
+  }
+  ldk::lds_barrier();
+  if (kg > 0) return;
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct) {
+    float mv[KG], lv[KG], M = m_run[ct];
+    mv[0] = m_run[ct];
+    lv[0] = l_w[ct];
+#pragma unroll
+    for (int g = 1; g < KG; ++g) {
+      mv[g] = mls[cg + g * CG][2 * ct][lane];
+      lv[g] = mls[cg + g * CG][2 * ct + 1][lane];
+      M = fmaxf(M, mv[g]);
+    }
+    float f[KG], l = 0.0f;
+#pragma unroll
+    for (int g = 0; g < KG; ++g) {
+      f[g] = mv[g] != -__builtin_inff() ? __builtin_amdgcn_exp2f((mv[g] - M) * sc) : 0.0f;
+      l = __builtin_fmaf(lv[g], f[g], l);
+    }
+    const int col = 32 * cg + 16 * ct + c16;
+    half_t* dst = out + (int64_t)(t0 + col) * ldo + (int64_t)h * kHD + 4 * kb;
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      float4_t v = o[ct][b] * f[0];
+#pragma unroll
+      for (int g = 1; g < KG; ++g) {
+        const float4_t w = red[((cg + (g - 1) * CG) * 16 + 8 * ct + b) * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = __builtin_fmaf(w[r], f[g], v[r]);
+      }
+      half4_t y;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[r] = (half_t)(l > 0.0f ? v[r] / l : 0.0f);
+      if (col < nt) *reinterpret_cast<half4_t*>(dst + 16 * b) = y;
+    }
   }
 }
 
@@ -864,10 +1213,38 @@ extern "C" int ldk_prefill_attention(const void* qkv, int64_t ldqkv, const int64
     return ldk::fail(LDK_ERR_ALIGN, "%s: k_cache, vt_cache and q_scratch 16-byte, pos 8-byte aligned", fn);
   hipStream_t s = (hipStream_t)stream;
   (void)hipGetLastError();
-  prefill_rope_kv_kernel<<<(unsigned)T, 256, 0, s>>>((const half_t*)qkv, ldqkv, pos, inv_freq, (half_t*)k_cache,
-                                                     (half_t*)vt_cache, (half_t*)q_scratch, nq, nkv, (int)max_len);
+  // heads split over workgroups until there are about three per CU (each forms its tokens' angles
+  // again: 2048 workgroups took 9.0 against 7.6 us at 3000 tokens of 12/2 heads)
+  const int64_t tb = (T + kRopeTok - 1) / kRopeTok;
+  const int hb = (int)std::min<int64_t>(nq + 2 * nkv, std::max<int64_t>(1, 768 / tb));
+  const bool vec = ldqkv % 8 == 0 && ldk::aligned(qkv, 16);
+  auto rope = [&](auto kernel) {
+    kernel<<<dim3((unsigned)tb, (unsigned)hb), 256, 0, s>>>((const half_t*)qkv, ldqkv, pos, (int)T, inv_freq, (half_t*)k_cache,
+                                                           (half_t*)vt_cache, (half_t*)q_scratch, nq, nkv, (int)max_len);
+  };
+  if (vec)
+    rope(prefill_rope_kv_kernel<true>);
+  else
+    rope(prefill_rope_kv_kernel<false>);
   int st = ldk::check_launch("prefill_rope_kv");
   if (st) return st;
+  // Blocks of tokens where they give the CUs enough workgroups. 128 tokens (one workgroup per CU)
+  // from 256 workgroups; 64 tokens in four K groups, which halve the longest workgroup's steps but
+  // load K and V twice as often, below (28/4 heads at 1500 tokens, 336 workgroups of 128: 51
+  // against 64 us; 16/16 at 816, 112: 39 against 36; 12/2 at 1024 after 3000, 96: 73 against 58).
+  // Under 128 workgroups of 64 the 16-token kernel's shorter start wins (12/2 at 511, 96
+  // workgroups: 20.2 against 21.9; at 128: 11.0 against 16.9 us). The block kernels divide by the
+  // scale (positive, not tiny) and store 8 bytes at a time.
+  auto launch_blocks = [&](auto kernel, int tokens) {
+    const dim3 grid((unsigned)nq, (unsigned)((T + tokens - 1) / tokens));
+    kernel<<<grid, 512, 0, s>>>((const half_t*)q_scratch, pos, (int)T, (const half_t*)k_cache, (const half_t*)vt_cache,
+                                (half_t*)out, ldo, nq, nkv, (int)max_len, scale);
+    return ldk::check_launch("prefill_attention");
+  };
+  if (scale > 1e-20f && ldo % 4 == 0 && ldk::aligned(out, 8) && (T + 63) / 64 <= 65535) {
+    if (nq * ((T + 127) / 128) >= 256) return launch_blocks(prefill_attention_block_kernel<4, 2, 4>, 128);
+    if (nq * ((T + 63) / 64) >= 128) return launch_blocks(prefill_attention_block_kernel<2, 4, 2>, 64);
+  }
   const dim3 grid((unsigned)((T + kTile - 1) / kTile), (unsigned)nq);
   prefill_attention_kernel<<<grid, kPWaves * 64, 0, s>>>((const half_t*)q_scratch, pos, (int)T, (const half_t*)k_cache,
                                                          (const half_t*)vt_cache, (half_t*)out, ldo, nq, nkv,

@@ -555,3 +555,54 @@ def test_prefill_cache_rows_past_the_prompt_can_hold_any_bits(p0, T):
     assert torch.isfinite(outs[0]).all()
     for o in outs[1:]:
         assert torch.equal(o, outs[0])
+
+
+@pytest.mark.parametrize("nq,nkv,L,p0,T", [(32, 8, 1056, 0, 1025), (64, 8, 2048, 700, 450), (64, 4, 1024, 31, 500),
+                                           (16, 16, 512, 0, 510), (32, 4, 1024, 33, 199), (70, 7, 160, 0, 100)])
+@pytest.mark.parametrize("order", ["in order", "shuffled"])
+def test_prefill_token_blocks_against_float64(nq, nkv, L, p0, T, order):
+    """ldk_prefill_attention on grids that take its blocks of 128 tokens (the first three: nq *
+    ceil(T / 128) >= 256) and of 64 (nq * ceil(T / 64) >= 128): one token and part of a tile in the
+    last block, prefixes that end inside a step, a cache shorter than a block's steps. Rows past
+    the prompt hold NaN, two tokens have positions outside the cache, and a row stride that is no
+    multiple of 8 takes the narrow loads. Float64 over the cache as stored; the bounds are
+    test_prefill_against_float64's, the k rows two fp16 roundings of |k| < 8 (2^-8)."""
+    from kernels.attention import prefill_attention
+
+    g = torch.Generator().manual_seed(p0 + 13 * T + nq)
+    hd, width = 128, (nq + 2 * nkv) * 128
+    narrow = order == "shuffled"
+    qkv = torch.randn(T, width + (2 if narrow else 0), generator=g).half().cuda()[:, :width]
+    kc, vc, _, _ = _caches(g, nkv, L)
+    kt, vt = _fill_past(kc, vc, p0 + T - 1, float("nan"))
+    inv = (1.0 / (1e6 ** (torch.arange(0, hd, 2, dtype=torch.float32) / hd))).cuda()
+    pos = torch.arange(p0, p0 + T, dtype=torch.int64)
+    if narrow:
+        pos = pos[torch.randperm(T, generator=g)]
+    pos = pos.cuda()
+    pos[T // 2] = -3
+    hole = int((set(range(p0, p0 + T)) - set(pos.tolist())).pop())  # not written: the cache's own row
+    out = prefill_attention(qkv.unsqueeze(0), pos, inv, kt, vt, nq, nkv, hd ** -0.5)[0].view(T, nq, hd)
+    k, v = k_from_tiles(kt)[0].double(), v_from_tiles(vt)[0].double()
+    assert torch.equal(k[:, hole].cpu(), kc[0, :, hole].double()) and torch.equal(v[:, hole].cpu(), vc[0, :, hole].double())
+    ang = (pos[:, None].float() * inv[None, :]).double()
+    cos, sin = torch.cat((ang, ang), -1).cos()[:, None], torch.cat((ang, ang), -1).sin()[:, None]
+
+    def rope(x):
+        return x * cos + torch.cat((-x[..., 64:], x[..., :64]), -1) * sin
+
+    x = qkv.double().view(T, -1, hd)
+    live = pos >= 0
+    assert (k[:, pos[live]] - rope(x[:, nq:nq + nkv])[live].transpose(0, 1)).abs().max() <= 2 ** -8
+    assert torch.equal(v[:, pos[live]], x[live, nq + nkv:].transpose(0, 1))
+    q = rope(x[:, :nq])
+    hidden = torch.arange(p0 + T, device="cuda")[None, :] > pos[:, None]
+    ref = torch.empty_like(q)
+    for h in range(nq):
+        kh, vh = k[h // (nq // nkv), :p0 + T], v[h // (nq // nkv), :p0 + T]
+        s = (q[:, h].contiguous() @ kh.t().contiguous()) * hd ** -0.5
+        ref[:, h] = torch.softmax(s.masked_fill(hidden, float("-inf")), -1) @ vh
+    ref[~live] = 0.0
+    err = (out.double() - ref).abs()
+    assert err.max() <= 2e-2 and err.norm() / ref.norm() <= 2e-3, (float(err.max()),)
+    assert torch.equal(out[~live], torch.zeros_like(out[~live]))
