@@ -23,25 +23,10 @@ namespace {
 
 // ------------------------------------------------------------------------------ e4m3 encode
 
-// float (|v| <= 448) -> e4m3fn byte, round to nearest, ties to even, sign of zero kept.
-// Written from the format: for |v| in [2^e, 2^(e+1)) with e >= -6 the spacing is 2^(e-3);
-// below 2^-6 (subnormal range) the spacing is 2^-9. Scaling by a power of two is exact, so
-// rintf on the scaled value performs the RNE rounding to the representable grid.
-__device__ __forceinline__ uint8_t e4m3_encode(float v) {
-  const uint32_t sign = (__builtin_bit_cast(uint32_t, v) >> 24) & 0x80u;
-  const float a = fabsf(v);
-  uint32_t code;
-  if (a < 0.015625f) {  // 2^-6
-    const uint32_t m = (uint32_t)rintf(a * 512.0f);  // 0..8; 8 is the smallest normal 2^-6
-    code = m;                                        // m == 8 encodes (e=1, m=0) = 0x08 as well
-  } else {
-    const int e = (int)((__builtin_bit_cast(uint32_t, a) >> 23) & 0xFF) - 127;  // -6..8
-    uint32_t m = (uint32_t)rintf(__builtin_ldexpf(a, 3 - e));                   // 8..16
-    int ee = e;
-    if (m == 16) { m = 8; ++ee; }
-    code = ((uint32_t)(ee + 7) << 3) | (m - 8);
-  }
-  return (uint8_t)(sign | code);
+// Two floats (|v| <= 448, no NaN) -> e4m3fn bytes in bits 7:0 and 15:8: gfx950's OCP conversion
+// rounds to nearest, ties to even, keeps the sign of zero and reaches the subnormals.
+__device__ __forceinline__ uint32_t e4m3_encode2(float a, float b) {
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false) & 0xffffu;
 }
 
 // e4m3fn byte -> float, written from the format (used where bit-exactness is the contract).
@@ -77,39 +62,165 @@ __device__ __forceinline__ uint16_t from_f32<uint16_t>(float v) {
   return (uint16_t)(u >> 16);
 }
 
-// One thread per output channel n: absmax over its row, then the row is quantized and written
-// as column n of wq. Consecutive threads take consecutive n, so each K step writes one
-// contiguous run of bytes. Arithmetic as fp8.py:27-29 in float32:
-// scale = max(absmax / 448, 1e-12); wq = e4m3(clamp(w / scale, -448, 448)).
-template <typename T>
-__global__ __launch_bounds__(64) void fp8_quantize_kernel(const T* __restrict__ w, uint8_t* __restrict__ wq,
-                                                          T* __restrict__ scale_out, int64_t N, int64_t K) {
-  const int64_t n = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (n >= N) return;
-  const T* row = w + n * K;
+// Quantizing takes three launches on one stream, because the absmax of a channel needs all of its
+// row and the output is the transposed layout:
+//  1. fp8_absmax_kernel, one workgroup per channel: absmax of its row, left in scale[n] (the largest
+//     of T's values is one of T's values, so nothing is lost there);
+//  2. fp8_quantize_kernel, tiles of 128 channels x 64 k turned through LDS: rows are read in
+//     128-byte runs and wq is written in 128-byte runs of one k row;
+//  3. fp8_scale_kernel: scale[n] = the rounded fp32 scale.
+// Arithmetic as fp8.py:27-29 in float32: scale = max(absmax / 448, 1e-12);
+// wq = e4m3(clamp(w / scale, -448, 448)). One thread per channel, reading its row twice, took
+// 1293 us on 14336 x 4096 fp16; this 59 us, of which the first launch is about 20.
+__device__ __forceinline__ float fp8_scale(float amax) { return fmaxf(amax / 448.0f, 1e-12f); }
+
+// V elements of T per load (1: any base and K).
+template <typename T, int V>
+__global__ __launch_bounds__(256) void fp8_absmax_kernel(const T* __restrict__ w, T* __restrict__ amax_out, int64_t K) {
+  typedef T tv_t __attribute__((ext_vector_type(V)));
+  __shared__ float part[4];
+  const T* row = w + (int64_t)blockIdx.x * K;
   float amax = 0.0f;
-  for (int64_t k = 0; k < K; ++k) amax = fmaxf(amax, fabsf(to_f32<T>(row[k])));
-  const float scale = fmaxf(amax / 448.0f, 1e-12f);
-  for (int64_t k = 0; k < K; ++k) {
-    const float q = fminf(fmaxf(to_f32<T>(row[k]) / scale, -448.0f), 448.0f);
-    wq[k * N + n] = e4m3_encode(q);
+  for (int64_t k = threadIdx.x * V; k < K; k += 256 * V) {
+    const tv_t v = *reinterpret_cast<const tv_t*>(row + k);
+#pragma unroll
+    for (int e = 0; e < V; ++e) amax = fmaxf(amax, fabsf(to_f32<T>(v[e])));
   }
-  scale_out[n] = from_f32<T>(scale);
+#pragma unroll
+  for (int o = 1; o < 64; o *= 2) amax = fmaxf(amax, __shfl_xor(amax, o));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;
+  __syncthreads();
+  if (threadIdx.x == 0) amax_out[blockIdx.x] = from_f32<T>(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void fp8_scale_kernel(T* __restrict__ scale, int64_t N) {
+  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (n < N) scale[n] = from_f32<T>(fp8_scale(to_f32<T>(scale[n])));
+}
+
+constexpr int kFCols = 128, kFRows = 64;  // channels and k of a tile
+
+// V: elements of T per load of w (8, or 1 for any base and K); S: bytes per store of wq (4 where the
+// k rows are 4-byte aligned, else 1).
+template <typename T, int V, int S>
+__global__ __launch_bounds__(256) void fp8_quantize_kernel(const T* __restrict__ w, const T* __restrict__ amax,
+                                                           uint8_t* __restrict__ wq, int64_t N, int64_t K) {
+  typedef T tv_t __attribute__((ext_vector_type(V)));
+  __shared__ __align__(4) uint8_t tile[kFRows][kFCols + 4];
+  const int64_t kt = (K + kFRows - 1) / kFRows;
+  const int64_t k0 = blockIdx.x % kt * kFRows, n0 = blockIdx.x / kt * kFCols;
+  constexpr int LPR = kFRows / V, P = kFCols * LPR / 256;  // lanes per channel, passes
+  constexpr int U = P < 8 ? P : 8;                         // loads in flight
+  const int tid = threadIdx.x, kk = tid % LPR * V;
+  for (int p0 = 0; p0 < P; p0 += U) {
+    tv_t v[U];
+    float sc[U];
+#pragma unroll
+    for (int p = 0; p < U; ++p) {  // channels past N and k past K repeat valid ones; not stored
+      const int64_t n = min(n0 + (p0 + p) * (256 / LPR) + tid / LPR, N - 1);
+      v[p] = *reinterpret_cast<const tv_t*>(w + n * K + min(k0 + kk, K - V));
+      sc[p] = fp8_scale(to_f32<T>(amax[n]));
+    }
+#pragma unroll
+    for (int p = 0; p < U; ++p) {
+      const int c = (p0 + p) * (256 / LPR) + tid / LPR;
+      // w / scale by the rounded reciprocal and two fma pairs, which round it correctly (as in the
+      // int4 quantizer, int4.hip) for any scale below 1e30; |w / scale| is at most about 448
+      const float y = 1.0f / sc[p];
+      const bool fast = __all(sc[p] < 1e30f);
+      uint32_t codes[(V + 1) / 2];
+      float q[V + 1];
+      q[V] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const float f = to_f32<T>(v[p][e]);
+        float d;
+        if (fast) {
+          d = f * y;
+          d = __builtin_fmaf(__builtin_fmaf(-sc[p], d, f), y, d);
+          d = __builtin_fmaf(__builtin_fmaf(-sc[p], d, f), y, d);
+          d = f == 0.0f ? f : d;  // -0 stays -0
+        } else {
+          d = f / sc[p];
+        }
+        q[e] = fminf(fmaxf(d, -448.0f), 448.0f);
+      }
+#pragma unroll
+      for (int e = 0; e < V; e += 2) codes[e / 2] = e4m3_encode2(q[e], q[e + 1]);
+#pragma unroll
+      for (int e = 0; e < V; ++e) tile[kk + e][c] = (uint8_t)(codes[e / 2] >> (8 * (e & 1)));
+    }
+  }
+  __syncthreads();
+  const int nn = tid * S % kFCols;
+  for (int r = tid * S / kFCols; r < kFRows; r += 256 * S / kFCols) {
+    if (k0 + r >= K || n0 + nn >= N) continue;
+    uint8_t* dst = wq + (k0 + r) * N + n0 + nn;
+    if constexpr (S == 4)
+      *reinterpret_cast<uint32_t*>(dst) = *reinterpret_cast<const uint32_t*>(&tile[r][nn]);
+    else
+      *dst = tile[r][nn];
+  }
 }
 
 // out [N, K] = (e4m3(wq[k, n]) * scale[n]) rounded once to the scale's dtype (fp8.py:33-35; the
-// product of an e4m3 value and an fp16/bf16 scale is exact in fp32).
-template <typename T>
+// product of an e4m3 value and an fp16/bf16 scale is exact in fp32). Tiles of 64 channels x 64 k
+// turned through LDS: a thread decodes 4 channels x 4 k and leaves each channel's 4 values as one
+// LDS write; an output row leaves in 16-byte stores (VS; one value each where the rows are not
+// 16-byte aligned). L: bytes per load (4 where the k rows are 4-byte aligned, else 1). One thread
+// per output, each reading a byte of its own line, took 236 us on 14336 x 4096 fp16 and 68 on
+// 1533 x 8960 bf16; this 47 and 17 (byte loads: the 4-byte ones need N % 4 == 0).
+template <typename T, int L, bool VS>
 __global__ __launch_bounds__(256) void fp8_dequant_kernel(const uint8_t* __restrict__ wq, const T* __restrict__ scale,
                                                           T* __restrict__ out, int64_t N, int64_t K) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= N * K) return;
-  const int64_t n = i / K, k = i - n * K;
-  float p = e4m3_decode(wq[k * N + n]) * to_f32<T>(scale[n]);
-  // Keep the f32 product: fused into one v_fma_mix with a +0 addend, the fp16 conversion would
-  // turn a -0 product (code 0x80) into +0.
-  asm volatile("" : "+v"(p));
-  out[i] = from_f32<T>(p);
+  typedef T t4_t __attribute__((ext_vector_type(4)));
+  constexpr int C = 64, E = 16 / sizeof(T);  // tile side, elements per 16-byte store
+  __shared__ __align__(16) T tile[C][C + E];
+  const int64_t kt = (K + C - 1) / C;
+  const int64_t k0 = blockIdx.x % kt * C, n0 = blockIdx.x / kt * C;
+  const int tid = threadIdx.x, c = tid % 16 * 4, kr = tid / 16 * 4;
+  uint32_t word[4];  // row kr + i: the bytes of channels c .. c + 3 (clamped ones are not stored)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint8_t* src = wq + min(k0 + kr + i, K - 1) * N;
+    if constexpr (L == 4) {  // N % 4 == 0
+      word[i] = *reinterpret_cast<const uint32_t*>(src + min(n0 + c, N - 4));
+    } else {
+      word[i] = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) word[i] |= (uint32_t)src[min(n0 + c + j, N - 1)] << (8 * j);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float sc = to_f32<T>(scale[min(n0 + c + j, N - 1)]);
+    t4_t v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float p = e4m3_decode((word[i] >> (8 * j)) & 0xFFu) * sc;
+      // Keep the f32 product: fused into one v_fma_mix with a +0 addend, the fp16 conversion would
+      // turn a -0 product (code 0x80) into +0.
+      asm volatile("" : "+v"(p));
+      v[i] = from_f32<T>(p);
+    }
+    *reinterpret_cast<t4_t*>(&tile[c + j][kr]) = v;
+  }
+  __syncthreads();
+  if constexpr (VS) {
+    typedef T tv_t __attribute__((ext_vector_type(E)));
+#pragma unroll
+    for (int i = 0; i < C * C / E / 256; ++i) {
+      const int t = tid + 256 * i, n = t / (C / E), k = t % (C / E) * E;
+      if (n0 + n < N && k0 + k < K)
+        *reinterpret_cast<tv_t*>(out + (n0 + n) * K + k0 + k) = *reinterpret_cast<const tv_t*>(&tile[n][k]);
+    }
+  } else {
+    for (int t = tid; t < C * C; t += 256) {
+      const int n = t / C, k = t % C;
+      if (n0 + n < N && k0 + k < K) out[(n0 + n) * K + k0 + k] = tile[n][k];
+    }
+  }
 }
 
 // --------------------------------------------------------------------------------- W8A16 GEMV
@@ -776,35 +887,72 @@ int launch_w8(const W8Args& a, const W8Split& sp, const W8Plan& p, hipStream_t s
 
 inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
+template <typename T>
+int launch_fp8_quantize(const T* w, uint8_t* wq, T* scale, int64_t N, int64_t K, hipStream_t s) {
+  const int64_t tiles = ((N + kFCols - 1) / kFCols) * ((K + kFRows - 1) / kFRows);
+  if (tiles > INT32_MAX || N > INT32_MAX) return ldk::fail(LDK_ERR_UNSUPPORTED, "fp8_quantize: too large");
+  const bool vec = K % 8 == 0 && ldk::aligned(w, 16), quad = N % 4 == 0 && ldk::aligned(wq, 4);
+  (void)hipGetLastError();
+  if (vec)
+    fp8_absmax_kernel<T, 8><<<(unsigned)N, 256, 0, s>>>(w, scale, K);
+  else
+    fp8_absmax_kernel<T, 1><<<(unsigned)N, 256, 0, s>>>(w, scale, K);
+  auto tile = [&](auto kernel) { kernel<<<(unsigned)tiles, 256, 0, s>>>(w, scale, wq, N, K); };
+  if (vec && quad)
+    tile(fp8_quantize_kernel<T, 8, 4>);
+  else if (vec)
+    tile(fp8_quantize_kernel<T, 8, 1>);
+  else if (quad)
+    tile(fp8_quantize_kernel<T, 1, 4>);
+  else
+    tile(fp8_quantize_kernel<T, 1, 1>);
+  fp8_scale_kernel<T><<<blocks_for(N, 256), 256, 0, s>>>(scale, N);
+  return ldk::check_launch("fp8_quantize");
+}
+
+template <typename T>
+int launch_fp8_dequant(const uint8_t* wq, const T* scale, T* out, int64_t N, int64_t K, hipStream_t s) {
+  const int64_t tiles = ((N + 63) / 64) * ((K + 63) / 64);
+  if (tiles > INT32_MAX) return ldk::fail(LDK_ERR_UNSUPPORTED, "fp8_dequant: too large");
+  const bool quad = N % 4 == 0 && ldk::aligned(wq, 4);
+  const bool vec = K * (int64_t)sizeof(T) % 16 == 0 && ldk::aligned(out, 16);
+  (void)hipGetLastError();
+  auto tile = [&](auto kernel) { kernel<<<(unsigned)tiles, 256, 0, s>>>(wq, scale, out, N, K); };
+  if (quad && vec)
+    tile(fp8_dequant_kernel<T, 4, true>);
+  else if (quad)
+    tile(fp8_dequant_kernel<T, 4, false>);
+  else if (vec)
+    tile(fp8_dequant_kernel<T, 1, true>);
+  else
+    tile(fp8_dequant_kernel<T, 1, false>);
+  return ldk::check_launch("fp8_dequant");
+}
+
 }  // namespace
 
 extern "C" int ldk_fp8_quantize(const void* w, int dtype, uint8_t* wq, void* scale, int64_t N, int64_t K, void* stream) {
   if (!w || !wq || !scale) return ldk::fail(LDK_ERR_INVALID, "fp8_quantize: null pointer");
   if (N <= 0 || K <= 0) return ldk::fail(LDK_ERR_INVALID, "fp8_quantize: N=%lld K=%lld must be positive", (long long)N, (long long)K);
   hipStream_t s = (hipStream_t)stream;
-  (void)hipGetLastError();
   switch (dtype) {
-    case LDK_F16: fp8_quantize_kernel<half_t><<<blocks_for(N, 64), 64, 0, s>>>((const half_t*)w, wq, (half_t*)scale, N, K); break;
-    case LDK_BF16: fp8_quantize_kernel<uint16_t><<<blocks_for(N, 64), 64, 0, s>>>((const uint16_t*)w, wq, (uint16_t*)scale, N, K); break;
-    case LDK_F32: fp8_quantize_kernel<float><<<blocks_for(N, 64), 64, 0, s>>>((const float*)w, wq, (float*)scale, N, K); break;
+    case LDK_F16: return launch_fp8_quantize((const half_t*)w, wq, (half_t*)scale, N, K, s);
+    case LDK_BF16: return launch_fp8_quantize((const uint16_t*)w, wq, (uint16_t*)scale, N, K, s);
+    case LDK_F32: return launch_fp8_quantize((const float*)w, wq, (float*)scale, N, K, s);
     default: return ldk::fail(LDK_ERR_INVALID, "fp8_quantize: unknown dtype %d", dtype);
   }
-  return ldk::check_launch("fp8_quantize");
 }
 
 extern "C" int ldk_fp8_dequant(const uint8_t* wq, const void* scale, int dtype, void* out, int64_t N, int64_t K, void* stream) {
   if (!wq || !scale || !out) return ldk::fail(LDK_ERR_INVALID, "fp8_dequant: null pointer");
   if (N <= 0 || K <= 0) return ldk::fail(LDK_ERR_INVALID, "fp8_dequant: N=%lld K=%lld must be positive", (long long)N, (long long)K);
   hipStream_t s = (hipStream_t)stream;
-  const unsigned g = blocks_for(N * K, 256);
-  (void)hipGetLastError();
   switch (dtype) {
-    case LDK_F16: fp8_dequant_kernel<half_t><<<g, 256, 0, s>>>(wq, (const half_t*)scale, (half_t*)out, N, K); break;
-    case LDK_BF16: fp8_dequant_kernel<uint16_t><<<g, 256, 0, s>>>(wq, (const uint16_t*)scale, (uint16_t*)out, N, K); break;
-    case LDK_F32: fp8_dequant_kernel<float><<<g, 256, 0, s>>>(wq, (const float*)scale, (float*)out, N, K); break;
+    case LDK_F16: return launch_fp8_dequant(wq, (const half_t*)scale, (half_t*)out, N, K, s);
+    case LDK_BF16: return launch_fp8_dequant(wq, (const uint16_t*)scale, (uint16_t*)out, N, K, s);
+    case LDK_F32: return launch_fp8_dequant(wq, (const float*)scale, (float*)out, N, K, s);
     default: return ldk::fail(LDK_ERR_INVALID, "fp8_dequant: unknown dtype %d", dtype);
   }
-  return ldk::check_launch("fp8_dequant");
 }
 
 // Rows from which the prefill GEMM (prefill.hip) replaces the MFMA kernel's 16-row blocks. The

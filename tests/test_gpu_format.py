@@ -157,3 +157,62 @@ def test_dequantize_column_sliced_scales_and_zeros():
     ref = dequantize_ref(np.ascontiguousarray(oqw[:, N:]), np.ascontiguousarray(os_[:, N:]),
                          np.ascontiguousarray(oz[:, N:]), 128)
     assert np.array_equal(bits16(out), bits16(ref))
+
+
+@pytest.mark.parametrize("N", [1, 63, 64, 65])
+@pytest.mark.parametrize("gs,K", [(32, 96), (64, 192), (128, 384), (256, 512), (512, 1024), (24, 48)])
+def test_quantize_rtn_column_tiles(N, gs, K):
+    """The tiled quantizer (groups of 32 .. 512, 64 columns per workgroup) at the edges of its
+    column tiles, and a group size that takes the general kernel; the last column's groups hold
+    infinities and a NaN, whose quotients divide, and ties of w / scale."""
+    w = (torch.randn(N, K, generator=cases.gen(N + gs)) * 0.05).half().numpy()
+    w[0] = (np.arange(K) % 31 - 15) * 0.25
+    if N > 1:
+        w[-1, 0], w[-1, gs], w[-1, gs + 1] = np.inf, -np.inf, np.nan
+    qw, s, z = quantize_rtn(dev(w), gs)
+    oqw, os_, oz = oq.quantize_rtn(w[:max(1, N - 1)], gs)
+    keep = slice(0, max(1, N - 1))
+    assert np.array_equal(to_np(qw)[:, keep], oqw)
+    assert np.array_equal(bits16(s)[:, keep], bits16(os_)) and np.array_equal(bits16(z)[:, keep], bits16(oz))
+    if N > 1:  # scale = inf: finite weights and inf / inf give 0 (a -inf makes the zero NaN)
+        assert to_np(qw)[: gs // 4, -1].max() == 0 and to_np(qw)[: gs // 4, -1].min() == 0
+
+
+def test_quantize_rtn_unaligned_weight():
+    """A weight whose base is not 16-byte aligned takes the general kernel; same bits."""
+    base = (torch.randn(70 * 256 + 3, generator=cases.gen(4)) * 0.05).half().cuda()
+    w = base[3:].view(70, 256)
+    for a, b in zip(quantize_rtn(w, 128), quantize_rtn(w.clone(), 128)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("N,K", [(1, 8), (63, 120), (64, 128), (65, 136), (130, 1032)])
+def test_dequantize_tiles(N, K):
+    """16 packed rows x 64 columns per workgroup, at the edges of both."""
+    g = cases.gen(N)
+    q = torch.randint(0, 16, (K, N), generator=g).int().numpy()
+    s = (torch.rand(K // 8, N, generator=g) * 0.1).half().numpy()
+    z = torch.randint(0, 16, (K // 8, N), generator=g).half().numpy()
+    out = dequantize(dev(oq.pack_int4(q)), dev(s), dev(z), 8)
+    assert np.array_equal(bits16(out), bits16(dequantize_ref(oq.pack_int4(q), s, z, 8)))
+
+
+@pytest.mark.parametrize("N", [1, 63, 64, 128, 132, 257])
+@pytest.mark.parametrize("K", [3, 64, 72, 129, 2056])
+def test_fp8_convert_tiles(N, K):
+    """quantize_fp8 (128 channels x 64 k per workgroup) and dequantize_fp8 (64 x 64) at the edges
+    of their tiles, with and without 4-byte aligned k rows and 16-byte aligned weight rows."""
+    from kernels.fp8 import dequantize_fp8, quantize_fp8
+    from oracle import fp8 as of
+
+    w = (torch.randn(N, K, generator=cases.gen(N + K)) * 0.05).half().numpy()
+    w[0, 0] = -0.0
+    wq, s = quantize_fp8(dev(w))
+    owq, os_ = of.quantize_fp8(w)
+    assert np.array_equal(wq.view(torch.uint8).cpu().numpy(), owq) and np.array_equal(bits16(s), bits16(os_))
+    assert np.array_equal(bits16(dequantize_fp8(wq, s)), bits16(of.dequantize_fp8(owq, os_)))
+    w32 = torch.from_numpy(w).float()
+    wq, s = quantize_fp8(w32.cuda())
+    owq, os_ = of.quantize_fp8(w32.numpy())
+    assert np.array_equal(wq.view(torch.uint8).cpu().numpy(), owq) and np.array_equal(to_np(s), os_)
+    assert np.array_equal(to_np(dequantize_fp8(wq, s)), of.dequantize_fp8(owq, os_))
