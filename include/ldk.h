@@ -275,7 +275,7 @@ int ldk_swiglu(const void* gate, int64_t ldg, const void* up, int64_t ldu, void*
  *   out:      [nq*head_dim] fp16; scale: the softmax scale (head_dim^-0.5).
  * head_dim == 128, nq % nkv == 0, max_len a multiple of 32 (k_cache and vt_cache 16-byte
  * aligned). A *pos >= max_len writes nothing and attends over the whole cache; a negative *pos
- * writes nothing and returns zeros. Caches of more than 512 positions are split into up to 32
+ * writes nothing and returns zeros. Caches of more than 512 positions are split into up to 128
  * position ranges whose partials go through library-owned device memory to a second launch on
  * the same stream that merges them (graph capture is safe); calls on one device must be
  * stream-ordered. warm, warm_bytes, nwarm: byte ranges the launch reads into the caches for the

@@ -9,7 +9,7 @@
 namespace ldk {
 
 constexpr int kAttnHeadDim = 128;  // head_dim of the decode attention
-constexpr int kAttnMaxSplits = 32;  // position ranges per head the partials hold
+constexpr int kAttnMaxSplits = 128;  // position ranges per head the partials hold
 constexpr int kAttnMaxHeads = 128;  // query heads the partials hold
 
 // Device addresses, on the current device, of the decode attention's per-range partials: `ml` is

@@ -18,7 +18,7 @@
 // Work split. One workgroup of NW waves (8; 4 where a range holds at most 4 chunks) serves up to
 // 16 query heads of one kv head (all of them for every GQA shape up to 16 heads per kv head), so
 // each K and V byte of a head is read once per launch, and its products run on the matrix cores
-// (v_mfma_f32_16x16x32_f16, the 16 heads are the tile's columns). Caches of more than 512 positions are cut into up to 32 position ranges
+// (v_mfma_f32_16x16x32_f16, the 16 heads are the tile's columns). Caches of more than 512 positions are cut into up to 128 position ranges
 // of at least 128 positions, with one workgroup per (head tile, range).
 //  - Wave w takes the 32-position chunks w, w + NW, ... of its range, two at a time, and loads
 //    each chunk's 8 K tiles and 8 V^T tiles (16 KB, all live) before its first use. The RoPE
@@ -67,6 +67,7 @@ constexpr int kChunk = 32;   // positions per score chunk and per P.V step
 constexpr int kBlock = 512;  // positions per softmax block: 16 chunks, two per wave
 constexpr int64_t kMaxLen = 1 << 20;
 constexpr int kMaxSplits = ldk::kAttnMaxSplits;  // position ranges per head tile
+constexpr int kRangesEntryMax = 32;  // of them, the most ldk_decode_attention_ranges takes
 constexpr int kMaxHeads = ldk::kAttnMaxHeads;    // query heads that can split (more run one range per tile)
 static_assert(kHD == ldk::kAttnHeadDim, "head_dim of the partials");
 constexpr uint32_t kDead = 0x80000000u;  // buffer offset past every resource: the load returns 0
@@ -455,41 +456,74 @@ __global__ __launch_bounds__(NW * 64) void decode_attention_kernel(AttnArgs a) {
   }
 }
 
-// The ranges' partials of one query head (one wave per head, launched after the ranges on the
-// same stream, so their stores are visible): lane r < nlive holds range r's (m, l); lane d reads
-// dims d and d + 64 of every live range's partial (coalesced dword loads, all in flight at once,
-// zero past the live ranges). With a single live range the range kernel has written the output
-// and this returns at once.
-__global__ __launch_bounds__(64) void attention_merge_kernel(const int64_t* pos_p, half_t* out, int L, int rlen) {
+// The ranges' partials of one query head (one workgroup per head, launched after the ranges on the
+// same stream, so their stores are visible). Every wave forms all the weights (lane r holds ranges
+// r and r + 64) and sums the ranges wave, wave + 8, ...: lane d reads dims 2d and 2d + 1 of each
+// live one's partial, all in flight at once, zero past the live ranges; the waves meet in LDS.
+// With a single live range the range kernel has written the output and this returns at once.
+constexpr int kMergeWaves = 8;
+
+__global__ __launch_bounds__(kMergeWaves * 64) void attention_merge_kernel(const int64_t* pos_p, half_t* out, int L,
+                                                                          int rlen) {
+  __shared__ float2_t part[kMergeWaves][kHD / 2];
   const int64_t pos_in = *pos_p;
   const bool pos_ok = pos_in >= 0 && pos_in < L;
   const int pos = pos_ok ? (int)pos_in : pos_in < 0 ? -1 : L - 1;
   const int nlive = pos < 0 ? 1 : pos / rlen + 1;
   if (nlive == 1) return;
-  const int h = blockIdx.x, lane = threadIdx.x;
-  const int r = min(lane, nlive - 1);
-  const float mr = g_ml[h][r][0], lr = g_ml[h][r][1];
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int RPW = kMaxSplits / kMergeWaves, RPL = kMaxSplits / 64;  // ranges per wave, per lane
+  float mr[RPL], lr[RPL];
+#pragma unroll
+  for (int i = 0; i < RPL; ++i) {
+    const int r = min(lane + 64 * i, nlive - 1);
+    mr[i] = g_ml[h][r][0];
+    lr[i] = g_ml[h][r][1];
+  }
   const auto ob = ldk::buffer_rsrc(&g_o[h][0][0], (uint32_t)sizeof(g_o[0]));
-  float ov0[kMaxSplits], ov1[kMaxSplits];
+  float2_t ov[RPW];
 #pragma unroll
-  for (int k = 0; k < kMaxSplits; ++k) {
-    const uint32_t off = (uint32_t)((k * kHD + lane) * 4) | (k < nlive ? 0u : kDead);
-    ov0[k] = ldk::u2f(__builtin_amdgcn_raw_buffer_load_b32(ob, off, 0, 0));
-    ov1[k] = ldk::u2f(__builtin_amdgcn_raw_buffer_load_b32(ob, off + 256, 0, 0));
+  for (int k = 0; k < RPW; ++k) {
+    const int r = wave + kMergeWaves * k;
+    const uint32_t off = (uint32_t)((r * kHD + 2 * lane) * 4) | (r < nlive ? 0u : kDead);
+    ov[k] = __builtin_bit_cast(float2_t, __builtin_amdgcn_raw_buffer_load_b64(ob, off, 0, 0));
   }
-  const float Mg = wave_max(lane < nlive ? mr : -__builtin_inff());
-  const float fr = lane < nlive ? __expf(mr - Mg) : 0.0f;  // weight of range `lane`
-  const float lg = ldk::sum_lanes_strided<1>(lr * fr);
-  float o0 = 0.0f, o1 = 0.0f;
+  float M = -__builtin_inff();
 #pragma unroll
-  for (int k = 0; k < kMaxSplits; ++k) {
-    // range k's weight, read into a scalar register (0 past the live ranges, whose loads read 0)
-    const float f = ldk::u2f(__builtin_amdgcn_readlane(ldk::f2u(fr), k));
-    o0 = __builtin_fmaf(ov0[k], f, o0);
-    o1 = __builtin_fmaf(ov1[k], f, o1);
+  for (int i = 0; i < RPL; ++i) M = fmaxf(M, lane + 64 * i < nlive ? mr[i] : -__builtin_inff());
+  M = wave_max(M);
+  float f[RPL], l = 0.0f;  // weights of this lane's ranges
+#pragma unroll
+  for (int i = 0; i < RPL; ++i) {
+    f[i] = lane + 64 * i < nlive ? __expf(mr[i] - M) : 0.0f;
+    l = __builtin_fmaf(lr[i], f[i], l);
   }
-  out[(int64_t)h * kHD + lane] = (half_t)(lg > 0.0f ? o0 / lg : 0.0f);
-  out[(int64_t)h * kHD + lane + 64] = (half_t)(lg > 0.0f ? o1 / lg : 0.0f);
+  l = ldk::sum_lanes_strided<1>(l);
+  float2_t o = {0.0f, 0.0f};
+#pragma unroll
+  for (int k = 0; k < RPW; ++k) {
+    // the range's weight, read into a scalar register (0 past the live ranges, whose loads read 0)
+    const int r = wave + kMergeWaves * k;
+    const float w = ldk::u2f(__builtin_amdgcn_readlane(ldk::f2u(f[k * kMergeWaves / 64]), r & 63));
+    o[0] = __builtin_fmaf(ov[k][0], w, o[0]);
+    o[1] = __builtin_fmaf(ov[k][1], w, o[1]);
+  }
+  part[wave][lane] = o;
+  __syncthreads();
+  if (wave) return;
+  float2_t v[kMergeWaves];
+#pragma unroll
+  for (int w = 0; w < kMergeWaves; ++w) v[w] = part[w][lane];
+  o = v[0];
+#pragma unroll
+  for (int w = 1; w < kMergeWaves; ++w) {
+    o[0] += v[w][0];
+    o[1] += v[w][1];
+  }
+  half_t* dst = out + (int64_t)h * kHD + 2 * lane;
+  dst[0] = (half_t)(l > 0.0f ? o[0] / l : 0.0f);
+  dst[1] = (half_t)(l > 0.0f ? o[1] / l : 0.0f);
 }
 
 // ------------------------------------------------------------ prompt (many-token) attention
@@ -1054,8 +1088,9 @@ extern "C" int ldk_decode_attention(const void* qkv, const int64_t* pos, const f
   // Position ranges: a cache of up to 512 positions runs one range (splitting it costs more in
   // the merge launch than it saves: 384 at pos 300 runs 7.9 us whole, 8.9 us in 128-position
   // ranges); longer ones at most kMaxSplits ranges of at least 128 positions (4096 at pos 4000:
-  // 9.5 us, 10.3 with 256-position ranges, 12.5 with 512). Caches with more heads than the
-  // partials hold run one range per head tile.
+  // 9.5 us, 10.3 with 256-position ranges, 12.5 with 512; 32768 in 128 ranges instead of 32: a
+  // 4-layer decode step at pos 6000 / 30000 207 / 211 -> 190 / 208 us). Caches with more heads than
+  // the partials hold run one range per head tile.
   const int64_t nblocks = (max_len + kBlock - 1) / kBlock;
   const int64_t nchunk = max_len / kChunk;
   int64_t rlen;
@@ -1082,7 +1117,7 @@ extern "C" int ldk_decode_attention(const void* qkv, const int64_t* pos, const f
   else
     decode_attention_kernel<8><<<nattn + nwg, 8 * 64, 0, (hipStream_t)stream>>>(a);
   if (nsplit > 1) {
-    attention_merge_kernel<<<nq, 64, 0, (hipStream_t)stream>>>(pos, (half_t*)out, (int)max_len, (int)rlen);
+    attention_merge_kernel<<<nq, kMergeWaves * 64, 0, (hipStream_t)stream>>>(pos, (half_t*)out, (int)max_len, (int)rlen);
     ldk::note_partials(false, stream, nullptr, 0, 0, 0);  // the partials of a pending range call are overwritten
   }
   return ldk::check_launch("decode_attention");
@@ -1104,9 +1139,9 @@ extern "C" int ldk_decode_attention_ranges(const void* qkv, const int64_t* pos, 
   if (max_len < kChunk || max_len > kMaxLen || max_len % kChunk)
     return ldk::fail(LDK_ERR_UNSUPPORTED, "decode_attention_ranges: max_len=%lld must be a multiple of 32 in 32..%lld",
                      (long long)max_len, (long long)kMaxLen);
-  if (rlen < kChunk || rlen % kChunk || rlen > max_len || (max_len + rlen - 1) / rlen > kMaxSplits)
+  if (rlen < kChunk || rlen % kChunk || rlen > max_len || (max_len + rlen - 1) / rlen > kRangesEntryMax)
     return ldk::fail(LDK_ERR_UNSUPPORTED, "decode_attention_ranges: rlen=%lld must be a multiple of 32 giving 1..%d ranges of %lld",
-                     (long long)rlen, kMaxSplits, (long long)max_len);
+                     (long long)rlen, kRangesEntryMax, (long long)max_len);
   if (!ldk::aligned(k_cache, 16) || !ldk::aligned(vt_cache, 16) || !ldk::aligned(pos, 8))
     return ldk::fail(LDK_ERR_ALIGN, "decode_attention_ranges: k_cache and vt_cache 16-byte, pos 8-byte aligned");
   const int nsplit = (int)((max_len + rlen - 1) / rlen);

@@ -474,6 +474,12 @@ class QwenRunner:
         self.vt_cache = torch.zeros((n, batch) + fa.vt_cache_shape(self.n_kv, max_len, d), device=dev, dtype=dt)
         self.keys = torch.arange(max_len, device=dev)
         self.merge_attention = True  # see forward: the o projection merges the attention's ranges
+        # Longest cache whose ranges the o projection merges: it takes at most four, so a range is a
+        # quarter of the cache, while decode_attention cuts it into up to 128 and merges them in a
+        # launch of its own. 4-layer decode steps (12/2 heads, W4A16), merged against split: cache
+        # 1024 at pos 371 175 / 182 us, 2048 at 1000 182 / 181, 4096 at 4000 196 / 181, 8192 at 6000
+        # 223 / 186, 32768 at 30000 387 / 208.
+        self.merge_max_len = 2048
         self.fuse_prompt_act = True  # see forward: SwiGLU in the prompt's gate_up GEMM
         self.warm_weights = True  # see warm_set: the attention launch warms the next weights
         self.fused_attention = (attention == "fused" and dev.type == "cuda"
@@ -565,7 +571,8 @@ class QwenRunner:
         prompt = self.fused_prefill and B == 1 and T > 1
         # the attention's ranges merged in the o projection's x staging (one launch fewer per
         # layer, and ranges of a quarter of the cache instead of one range per kv head)
-        merge = fused and self.merge_attention and be.merges_attention
+        merge = (fused and self.merge_attention and be.merges_attention
+                 and self.max_len <= self.merge_max_len)
         if merge:
             from kernels.attention import MERGE_MAX_RANGES, decode_attention_ranges, ranges_len
 

@@ -606,3 +606,27 @@ def test_prefill_token_blocks_against_float64(nq, nkv, L, p0, T, order):
     err = (out.double() - ref).abs()
     assert err.max() <= 2e-2 and err.norm() / ref.norm() <= 2e-3, (float(err.max()),)
     assert torch.equal(out[~live], torch.zeros_like(out[~live]))
+
+
+@pytest.mark.parametrize("nq,nkv,L,pos", [(12, 2, 8192, 8191), (12, 2, 8192, 128), (32, 8, 16416, 16300),
+                                          (28, 4, 40000, 39999), (12, 2, 40000, 20000)])
+def test_decode_attention_many_ranges_against_float64(nq, nkv, L, pos):
+    """ldk_decode_attention on caches cut into more than 32 ranges: 64 of 128 positions, 103 of 160 and
+    125 of 320 (the last one short), with one range live past the first, about half and all of them.
+    Float64 over the cache as stored; the bounds of the shorter caches' test."""
+    g = torch.Generator().manual_seed(pos + nq)
+    hd = 128
+    qkv = torch.randn((nq + 2 * nkv) * hd, generator=g).half().cuda()
+    _, _, kt, vt = _caches(g, nkv, L)
+    inv = (1.0 / (1e6 ** (torch.arange(0, hd, 2, dtype=torch.float32) / hd))).cuda()
+    out = decode_attention(qkv.view(1, 1, -1), torch.tensor([pos], device="cuda"), inv, kt, vt, nq, nkv, hd ** -0.5)
+    k, v = k_from_tiles(kt)[0, :, :pos + 1].double(), v_from_tiles(vt)[0, :, :pos + 1].double()
+    x = qkv.double().view(-1, hd)
+    assert torch.equal(v[:, pos], x[nq + nkv:])
+    ang = (torch.tensor(float(pos), device="cuda") * inv).double()
+    cos, sin = torch.cat((ang, ang)).cos(), torch.cat((ang, ang)).sin()
+    q = x[:nq] * cos + torch.cat((-x[:nq, 64:], x[:nq, :64]), -1) * sin
+    s = torch.matmul(q.view(nkv, nq // nkv, hd), k.transpose(1, 2).contiguous()) * hd ** -0.5
+    ref = torch.matmul(torch.softmax(s, -1), v).view(1, 1, -1)
+    err = (out.double() - ref).abs()
+    assert err.max() <= 2e-2 and err.norm() / ref.norm() <= 2e-3, (float(err.max()),)
