@@ -525,7 +525,8 @@ __global__ __launch_bounds__(NW * 64) void w8a16_gemv_kernel(W8Args a, W8Split s
 //    is the real column n0 + 8 c16 + j).
 //  * A operand: x row m = c16, K block 8 kb, one 16-byte load (zeros past M or past K).
 // A workgroup owns 128 columns and a K range; its waves take K steps round-robin, KSW per pass
-// with every load of the pass in flight; partial tiles meet in LDS, then the per-channel scale.
+// with every load of the pass in flight (PIPE: and the next pass's); partial tiles meet in LDS,
+// then the per-channel scale.
 // 64-column tiles share each 128-byte line of a K row with their neighbour. A lane's CPL-byte
 // loads need rows aligned to CPL bytes: N % 8 == 0 for 128 columns, N % 4 == 0 for 64 (the plan
 // takes 64 when N % 8 != 0). Their launch is one
@@ -549,7 +550,7 @@ __device__ __forceinline__ void w8_pair_piece(int b, int tiles, int& tile, int& 
   }
 }
 
-template <int NW, int KSW, int CW>
+template <int NW, int KSW, int CW, bool PIPE>
 __global__ __launch_bounds__(NW * 64) void w8a16_mfma_kernel(W8Args a, W8Split sp) {
   typedef _Float16 half8v __attribute__((ext_vector_type(8)));
   static_assert(CW == 128 || CW == 64, "128 or 64 columns");
@@ -575,22 +576,29 @@ __global__ __launch_bounds__(NW * 64) void w8a16_mfma_kernel(W8Args a, W8Split s
 #pragma unroll
   for (int j = 0; j < CPL; ++j) acc[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-  for (int s0 = wave; s0 < nks; s0 += NW * KSW) {
+  // KSW K steps of this wave from step s0 on (every NW-th): all their loads, then their products
+  struct Buf {
     wrow_t w[KSW][8];
     u32x4 xa[KSW];
+  };
+  auto load = [&](Buf& b, int s0) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < KSW; ++u) {
       const int kblk = rb + (s0 + u * NW) * 32 + 8 * kb;  // first of this lane's 8 rows
       const bool kok = s0 + u * NW < nks && kblk < re;
-      xa[u] = *reinterpret_cast<const u32x4*>(xrow + min(kblk, a.K - 8));
-      if (!kok || !xrow_ok) xa[u] = u32x4{0u, 0u, 0u, 0u};
+      b.xa[u] = *reinterpret_cast<const u32x4*>(xrow + min(kblk, a.K - 8));
+      if (!kok || !xrow_ok) b.xa[u] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int r = min(kblk + i, re - 1);
-        w[u][i] = __builtin_nontemporal_load(reinterpret_cast<const wrow_t*>(a.wq + (int64_t)r * a.N + col));
+        b.w[u][i] = __builtin_nontemporal_load(reinterpret_cast<const wrow_t*>(a.wq + (int64_t)r * a.N + col));
       }
     }
     __builtin_amdgcn_sched_barrier(0);  // every load of the pass is in flight before the first wait
+  };
+  auto multiply = [&](const Buf& b, int s0) __attribute__((always_inline)) {
+    const auto& w = b.w;
+    const auto& xa = b.xa;
 #pragma unroll
     for (int u = 0; u < KSW; ++u) {
       if (s0 + u * NW >= nks) break;  // uniform
@@ -623,6 +631,27 @@ __global__ __launch_bounds__(NW * 64) void w8a16_mfma_kernel(W8Args a, W8Split s
         }
         acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, __builtin_bit_cast(half8v, b), acc[j], 0, 0, 0);
       }
+    }
+  };
+  if constexpr (PIPE) {
+    // the loads of the next KSW steps are in flight while these multiply (steps past the range load
+    // its last row again and are not multiplied)
+    constexpr int D = NW * KSW;
+    Buf b0, b1;
+    load(b0, wave);
+    for (int s0 = wave; s0 < nks; s0 += 2 * D) {
+      load(b1, s0 + D);
+      multiply(b0, s0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(b0, s0 + 2 * D);
+      multiply(b1, s0 + D);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    for (int s0 = wave; s0 < nks; s0 += NW * KSW) {
+      Buf b;
+      load(b, s0);
+      multiply(b, s0);
     }
   }
 
@@ -664,6 +693,7 @@ struct W8Plan {
   int64_t words;  // split-K accumulator words (one per output of every tile and row block)
   bool mfma;
   int ksw;  // MFMA kernel: 32-row K steps per wave and pass
+  bool pipe;  // MFMA kernel: a pass's loads go out before the products of the one before
 };
 
 constexpr int kW8MfmaWaves = 8;
@@ -709,12 +739,28 @@ W8Plan make_w8_mfma_plan(int64_t M, int64_t N, int64_t K, int block_n, int split
   // 64-column tiles load 4 (N % 4 == 0). Prefill rows of short K take 64 columns too.
   p.ln = block_n == 64 || (block_n == 0 && (narrow || N % 8 || (M > 16 && w8_short_k(K)))) ? 4 : 8;
   p.nw = kW8MfmaWaves;
-  const int64_t tiles = (N + 16 * p.ln - 1) / (16 * p.ln);
   const int64_t steps = (K + 31) / 32;
+  // Decode rows over 20 MB of weights or more whose K takes a wave more than one pass: 128-column
+  // tiles, K split only as far as one workgroup per CU. A piece then streams long enough that its
+  // start and its returning atomics (one per output and split) weigh little: M = 2 / 13, against the
+  // plans below, 28672x4096 in 1 split (8 / 3 before) 27.5 / 38.9 -> 24.7 / 27.6 us, 4096x14336 in 8
+  // (10 of 64 columns) 20.8 / 28.4 -> 13.8 / 18.2, 11264x2048 in 2 (4 / 2 of 64) 9.7 / 12.9 -> 8.1 /
+  // 11.2; under 14 MB the plans below win (1536x8960 in 10 of 64 6.2 / 7.2 against 7.4 / 9.9). From 5
+  // rows at most 8 splits (3072x7680 in 10: M = 13 12.1 against 11.7 us in 5 of 64 columns); up to 4
+  // rows not where whole tiles would leave a quarter of the CUs idle and the pieces of 16 steps
+  // below do not (20480x2560, 160 tiles: 16.9 against 15.0).
+  const int64_t wide_tiles = (N + 127) / 128, wide_splits = std::max<int64_t>(1, std::min<int64_t>(256 / wide_tiles, steps / 8));
+  const bool stream = M <= 16 && block_n == 0 && split_k <= 0 && N % 8 == 0 && steps > 48 && wide_tiles <= 256 &&
+                      N * K >= 20000000 &&
+                      (M <= 4 ? wide_tiles < 128 || wide_tiles * wide_splits >= 192 : wide_splits <= 8);
+  if (stream) p.ln = 8;
+  const int64_t tiles = (N + 16 * p.ln - 1) / (16 * p.ln);
   const int64_t one_pass = (steps + 6 * p.nw - 1) / (6 * p.nw);  // fewest splits of one pass each
   int64_t splits;
   if (split_k > 0) {
     splits = split_k;
+  } else if (stream) {
+    splits = wide_splits;
   } else if (tiles >= 128 && M <= 4) {  // pieces of 16 steps: gate_up M = 2 / 3 / 4 in three,
                                         // 8.76 / 8.83 / 8.73 -> 7.91 / 8.11 / 8.39 us (at 5 rows
                                         // and more the pieces' atomics cost more than they save)
@@ -748,11 +794,16 @@ W8Plan make_w8_mfma_plan(int64_t M, int64_t N, int64_t K, int block_n, int split
   if (p.ln == 4 && M > 16 && p.splits > 1 && w8_short_k(K)) p.nw = kW8MfmaWavesWide;
   const int64_t per_wave = ((p.kps / 32) + p.nw - 1) / p.nw;
   // K steps per wave and pass: 16 waves hold at most 4 each in registers (1024 lanes: 128 VGPRs)
-  p.ksw = per_wave <= 1 ? 1 : per_wave <= 2 ? 2 : (per_wave <= 4 || p.nw == kW8MfmaWavesWide) ? 4 : 6;
+  // more than one pass per wave on 128-column tiles: two steps a pass, the next pass's loads ahead
+  // (28672x4096 whole K, M = 2 / 8 / 16: 26.7 / 27.7 / 29.6 -> 24.7 / 26.1 / 28.4 us; 4096x14336 in 8
+  // splits 15.6 / 17.6 / 20.5 -> 13.8 / 16.1 / 18.5; three or four steps a pass are no faster than six
+  // unpipelined ones)
+  p.pipe = p.ln == 8 && per_wave > 6;
+  p.ksw = p.pipe ? 2 : per_wave <= 1 ? 1 : per_wave <= 2 ? 2 : (per_wave <= 4 || p.nw == kW8MfmaWavesWide) ? 4 : 6;
   return p;
 }
 
-template <int NW, int KSW, int CW>
+template <int NW, int KSW, int CW, bool PIPE = false>
 int launch_w8_mfma_t(const W8Args& a, const W8Split& sp, hipStream_t s) {
   const unsigned tiles = (unsigned)((a.N + CW - 1) / CW), blocks = (unsigned)((a.M + 15) / 16);
   // 64-column tiles: one dimension over (tile, split) pieces (w8_pair_piece)
@@ -760,7 +811,7 @@ int launch_w8_mfma_t(const W8Args& a, const W8Split& sp, hipStream_t s) {
   const size_t lds = (size_t)NW * 16 * CW * 4;
   static_assert((size_t)NW * 16 * CW * 4 <= 64 * 1024, "the LDS reduction fits the default dynamic LDS limit");
   (void)hipGetLastError();
-  w8a16_mfma_kernel<NW, KSW, CW><<<grid, NW * 64, lds, s>>>(a, sp);
+  w8a16_mfma_kernel<NW, KSW, CW, PIPE><<<grid, NW * 64, lds, s>>>(a, sp);
   return ldk::check_launch("w8a16_mfma");
 }
 
@@ -776,6 +827,8 @@ int launch_w8_mfma_cw(const W8Args& a, const W8Split& sp, const W8Plan& p, hipSt
       return ldk::fail(LDK_ERR_UNSUPPORTED, "w8a16: %d K steps per wave not instantiated for 16 waves", p.ksw);
     }
   }
+  if constexpr (CW == 128)
+    if (p.pipe) return launch_w8_mfma_t<kW8MfmaWaves, 2, CW, true>(a, sp, s);
   if (p.nw != kW8MfmaWaves) return ldk::fail(LDK_ERR_UNSUPPORTED, "w8a16: %d waves not instantiated", p.nw);
   switch (p.ksw) {
     case 1: return launch_w8_mfma_t<kW8MfmaWaves, 1, CW>(a, sp, s);

@@ -385,3 +385,23 @@ def test_prefill_row_blocks_one_hot_rows_exact():
     ref = of.e4m3_decode(codes[ks.numpy()]).astype(np.float16)
     assert np.array_equal(bits16(to_np(out)) & 0x7FFF | (bits16(ref) & 0x8000) * (ref != 0),
                           bits16(ref) & 0x7FFF | (bits16(ref) & 0x8000) * (ref != 0))
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 1536, 14344), (5, 28680, 1576), (13, 11272, 1800), (16, 4096, 14336),
+                                   (16, 28672, 1576)])
+def test_decode_rows_on_large_weights(M, N, K):
+    """Decode rows over at least 20 MB of e4m3 weights: 128-column tiles with at most one workgroup
+    per CU, K split or whole, one pass per wave or pipelined passes, with the last tile and the last
+    K step partial. Against float64 on the GPU at the suite's matmul bounds."""
+    from kernels.fp8 import config_for
+
+    tiles = -(-N // 128)
+    assert config_for(M, N, K) == f"mfma,block_n=128,split_k={max(1, 256 // tiles)}"
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.02).half()
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    b = torch.randn(N, generator=g, device="cuda").half()
+    wq, s = quantize_fp8(w)
+    y = w8a16_matmul(x, wq, s, bias=b).double()
+    ref = x.double() @ (wq.float().double() * s.double()).contiguous() + b.double()
+    assert (y - ref).abs().max() <= 2e-2 and (y - ref).norm() / ref.norm() <= 1e-3
