@@ -1395,7 +1395,15 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int gsh_rows, int block_n, int s
   // Two rows on a narrow shape of more than 2 MB (down) also take the MFMA kernel, split K ten
   // ways: 4.9 against 5.4 us for the two-row VALU kernel (wide shapes keep it: gate_up 5.7 us).
   const bool narrow_long = N < 128 * 128 && wbytes > (2 << 20);
-  const bool mfma_auto = M > 8 || (!(flags & LDK_EXACT) && (M > 2 || (M == 2 && narrow_long && block_n == 0)) &&
+  // One and two rows take the MFMA kernel from 48M weights: the VALU kernels' tiles of 32 columns
+  // over a long K then run in several rounds of workgroups (M = 1 / 2: 28672x4096 17.0 / 18.3 ->
+  // 15.4 / 15.4 us, 14336x4096 11.0 / 11.6 -> 8.6 / 8.6, 4096x14336 M = 1 12.4 -> 9.1; 6144x4096, 25M
+  // weights, 5.6 against 6.1), unless its 64-column tiles leave a quarter of the CUs idle (10240x8192,
+  // 160 tiles, M = 1 12.4 against 13.5).
+  const int64_t t64 = (N + 63) / 64;
+  const bool few_large = M <= 2 && N * K >= 48000000 && block_n == 0 && split_k <= 0 && !(flags & LDK_FACTORED) &&
+                         (M == 2 || t64 > 256 || t64 * (256 / t64) >= 192);
+  const bool mfma_auto = M > 8 || (!(flags & LDK_EXACT) && (M > 2 || (M == 2 && narrow_long && block_n == 0) || few_large) &&
                                    (block_n == 0 || block_n >= 64));
   const bool mfma = (flags & LDK_PATH_MFMA) || (mfma_auto && !(flags & LDK_PATH_VALU));
   const bool m1 = !mfma && !(flags & LDK_EXACT) && M <= 2;  // the factored VALU kernel
@@ -1427,6 +1435,14 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int gsh_rows, int block_n, int s
   }
   p.mt = mfma ? 16 : round_mt(M);
   p.mtile = mfma && M > 16 ? 2 : 1;
+  // Decode rows from 20M weights: 64-column tiles where they number at most 256, K split only as far
+  // as one workgroup per CU. M = 4 / 16, against the plans below: 6144x4096 in 2 splits (3 of 64
+  // columns, 288 workgroups; 32 columns) 8.2 / 8.1 -> 6.2 / 7.8 us, 14336x4096 whole (32 columns from 13
+  // rows) 8.8 / 15.1 -> 8.8 / 10.6, 4096x14336 in 4 9.2 / 23.1 -> 9.1 / 11.2, 2560x11648 in 6 M = 16
+  // 9.5 -> 8.3, 8192x8192 in 2 12.5 / 13.5 -> 9.8 / 11.6; from 13 rows not where a short K would be
+  // split (8064x2560 in 2 7.2 against 6.5).
+  const bool large = mfma && M <= 16 && block_n == 0 && split_k <= 0 && N * K >= 20000000 && t64 <= 256 &&
+                     (M <= 12 || K >= 4096 || t64 > 128);
   if (mfma) {  // 128 columns on shapes wide enough to fill the CUs with them, else 64 (and 64 for
               // 32-row blocks of group-256 weights, whose 128-column variant runs out of registers);
               // decode rows on shapes of <= 2 MB take 32 columns (q/o/k/v at M = 8: 4.7 -> 4.4 us),
@@ -1435,6 +1451,7 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int gsh_rows, int block_n, int s
     p.ln = block_n == 32    ? 8
            : block_n == 64  ? 16
            : block_n == 128 ? 32
+           : large          ? 16
            : (M <= 16 && wbytes <= (2 << 20)) ? 8
            : (M > 12 && M <= 16 && N < 128 * 128 && split_k <= 0) ? 8
            : (N >= 128 * 128 && !(M > 16 && rpg > 16) ? 32 : 16);
@@ -1466,6 +1483,7 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int gsh_rows, int block_n, int s
   // 8 / 16 in 10 splits 4.9 / 5.0 / 5.45 / 6.70 us, in 8 splits 5.2 / 5.2 / 5.6 / 6.73)
   if (split_k <= 0 && tiles < 128 && wbytes > (2 << 20) && M <= 16)
     splits = m1 ? std::max<int64_t>(2, 256 / tiles) : (240 + tiles - 1) / tiles;
+  if (large) splits = std::max<int64_t>(1, 256 / tiles);
   // Prefill rows in row blocks of 32 (mtile 2, at most 8 waves) or 16 (mtile 1, up to 16 waves).
   // A long-K shape whose tiles and blocks leave most CUs idle splits K toward 256 workgroups, at
   // most 8 ways and never past 256 (a CU with two finishes last: down 1536x8960 M = 128 in 32-row
@@ -2147,7 +2165,7 @@ extern "C" int ldk_w4a16_rmsnorm_matmul(const void* x, const void* residual, voi
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_rmsnorm_matmul: norm_weight, residual and residual_out must be 16-byte aligned");
   if (workspace_bytes && (!workspace || !ldk::aligned(workspace, 256)))
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_rmsnorm_matmul: workspace must be a 256-byte aligned pointer");
-  Plan p = make_plan(1, N, K, gsh_rows, 0, 0, 0, workspace ? (size_t)workspace_bytes : 0);
+  Plan p = make_plan(1, N, K, gsh_rows, 0, 0, LDK_PATH_VALU, workspace ? (size_t)workspace_bytes : 0);
   if (p.full) {  // whole tiles: every workgroup then reads the whole row, which its statistic needs
     p.full = 0;
     p.splits = 1;
@@ -2167,7 +2185,7 @@ extern "C" int ldk_w4a16_swiglu_matmul(const void* gate_up, const int32_t* qweig
   if (st) return st;
   if (workspace_bytes && (!workspace || !ldk::aligned(workspace, 256)))
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_swiglu_matmul: workspace must be a 256-byte aligned pointer");
-  const Plan p = make_plan(1, N, K, gsh_rows, 0, 0, 0, workspace ? (size_t)workspace_bytes : 0);
+  const Plan p = make_plan(1, N, K, gsh_rows, 0, 0, LDK_PATH_VALU, workspace ? (size_t)workspace_bytes : 0);
   const W4Args a{(const half_t*)gate_up, 2 * K, (const uint32_t*)qweight, (const half_t*)scales, (const half_t*)zeros,
                  (const half_t*)bias, (half_t*)out, N, 1, (int)N, (int)K, gsh_rows};
   return launch_plan(a, p, workspace, (hipStream_t)stream, kProSwiglu, ProArgs{});
@@ -2183,7 +2201,7 @@ extern "C" int ldk_w4a16_swiglu_matmul(const void* gate_up, const int32_t* qweig
 
 namespace {
 Plan residual_stats_plan(int64_t N, int64_t K, int gsh_rows, size_t ws) {
-  Plan p = make_plan(1, N, K, gsh_rows, 0, 0, 0, ws);
+  Plan p = make_plan(1, N, K, gsh_rows, 0, 0, LDK_PATH_VALU, ws);
   p.full = 0;
   p.splits = 1;
   p.gps = (int)((K / 8) >> gsh_rows);
@@ -2280,7 +2298,7 @@ extern "C" int ldk_w4a16_rmsnorm_stats_matmul(const void* h, const float* row_st
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_rmsnorm_stats_matmul: norm_weight 16-byte, row_stats 4-byte aligned");
   if (workspace_bytes && (!workspace || !ldk::aligned(workspace, 256)))
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_rmsnorm_stats_matmul: workspace must be a 256-byte aligned pointer");
-  const Plan p = make_plan(1, N, K, gsh_rows, 0, 0, 0, workspace ? (size_t)workspace_bytes : 0);
+  const Plan p = make_plan(1, N, K, gsh_rows, 0, 0, LDK_PATH_VALU, workspace ? (size_t)workspace_bytes : 0);
   const W4Args a{(const half_t*)h, K, (const uint32_t*)qweight, (const half_t*)scales, (const half_t*)zeros,
                  (const half_t*)bias, (half_t*)out, N, 1, (int)N, (int)K, gsh_rows};
   const ProArgs pa{nullptr, nullptr, (const half_t*)norm_weight, eps, const_cast<float*>(row_stats), nstats};

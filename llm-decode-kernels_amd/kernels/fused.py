@@ -24,10 +24,14 @@ from kernels.w4a16 import w4a16_matmul
 FUSED_GROUP_SIZE = 128
 # Widest projection that rmsnorm_w4a16_matmul fuses. Every workgroup of the fused launch forms
 # the row statistic itself (its own loads and a barrier) and the launch takes whole column tiles,
-# which costs little on one round of tiles and grows with the rounds: graph-timed at K = 1536,
-# N = 2048 3.46 against 3.37 us plain, N = 17920 7.52 against 5.25, and the 151936-row quantized
-# lm_head 33.4 against 24.0 us, where the norm as a launch of its own (about 2.5 us) wins.
-FUSED_NORM_MAX_N = 65536
+# which costs little on one round of tiles and grows with the rounds. Graph-timed, fused against
+# the norm as a launch of its own: 2048x1536 3.6 / 5.5 us, 17920x1536 7.4 / 7.5, 18688x2176
+# 10.9 / 10.0, 28672x4096 24.2 / 17.8, the 151936-row quantized lm_head 33.4 / 26.5.
+FUSED_NORM_MAX_N = 18432
+# Weights (N * K) from which one row's projection runs the library's matrix-core plan, which takes
+# no prologue: the norm or activation is then a launch of its own (swiglu into 4096x14336 12.7 us
+# fused, 11.0 in two launches; 2560x11648, 30M weights, 6.4 against 8.1).
+FUSED_MAX_WEIGHTS = 48_000_000
 
 
 def _aligned(*ts) -> bool:
@@ -45,6 +49,7 @@ def rmsnorm_w4a16_matmul(x, weight, eps, residual, qweight, scales, zeros, group
     rows = x.numel() // K
     fuse = (rows == 1 and group_size == FUSED_GROUP_SIZE and x.dtype == torch.float16
             and weight.dtype == torch.float16 and x.is_cuda and N <= FUSED_NORM_MAX_N
+            and N * K < FUSED_MAX_WEIGHTS
             and _aligned(x, weight, residual, qweight))
     if not fuse:
         if residual is None:
@@ -80,7 +85,8 @@ def swiglu_w4a16_matmul(gate_up, qweight, scales, zeros, group_size=128, bias=No
     N = qweight.shape[1]
     rows = gate_up.numel() // K2
     fuse = (rows == 1 and group_size == FUSED_GROUP_SIZE and gate_up.dtype == torch.float16
-            and gate_up.is_cuda and _aligned(gate_up, qweight) and K % 8 == 0)
+            and gate_up.is_cuda and _aligned(gate_up, qweight) and K % 8 == 0
+            and N * K < FUSED_MAX_WEIGHTS)
     if not fuse:
         return w4a16_matmul(swiglu_fused(gate_up), qweight, scales, zeros, group_size, bias)
     assert K2 % 2 == 0 and qweight.shape[0] * 8 == K

@@ -10,6 +10,7 @@ import torch
 from _util import assert_north_star, bits16, dev, to_np
 from kernels.bench import cases
 from kernels.cuda.w4a16_cuda import w4a16_decode_cuda
+from kernels.quant import pack_int4
 from kernels.w4a16 import config_for, kernel_name, w4a16_matmul
 from oracle import quant as oq
 from oracle.reference import dequantize_ref, w4a16_ref
@@ -657,3 +658,24 @@ def test_prefill_16_row_blocks_one_hot_rows_exact(N, K):
     out = w4a16_matmul(dev(x), dev(qw), dev(s), dev(z))
     deq = dequantize_ref(qw, s, z)
     assert np.array_equal(bits16(out), bits16(deq[:, ks].T))
+
+
+@pytest.mark.parametrize("M,N,K,plan", [(1, 14340, 4096, "mfma,block_n=64,split_k=1"), (2, 28676, 1792, "mfma,block_n=128,split_k=1"),
+                                        (5, 6148, 4096, "mfma,block_n=64,split_k=2"), (16, 8192, 8192, "mfma,block_n=64,split_k=2"),
+                                        (13, 1036, 20480, "mfma,block_n=64,split_k=15")])
+def test_decode_rows_on_large_weights(M, N, K, plan):
+    """Decode rows over 20M int4 weights (48M for one and two rows): 64-column tiles on at most one
+    workgroup per CU, whole K or split, with a partial last tile. Against float64 on the GPU at the
+    suite's relative bound, and 5e-3 of max(1, |y|) elementwise (ten fp16 roundings of the output)."""
+    assert config_for(M, N, K).startswith(plan)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    q = torch.randint(0, 16, (K, N), generator=g, device="cuda").int()
+    s = (torch.rand(K // 128, N, generator=g, device="cuda") * 0.004 + 0.002).half()
+    z = torch.randint(6, 10, (K // 128, N), generator=g, device="cuda").half()
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    packed = pack_int4(q)
+    y = w4a16_matmul(x, packed, s, z).double()
+    w = ((q.double().view(K // 128, 128, N) - z.double()[:, None]) * s.double()[:, None]).view(K, N)
+    ref = x.double() @ w
+    # the dequantized weight is rounded to fp16 nowhere in the factored form: fp32 sums, one rounding
+    assert (y - ref).norm() / ref.norm() <= 1e-3 and ((y - ref).abs() / ref.abs().clamp_min(1.0)).max() <= 5e-3
