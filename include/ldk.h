@@ -193,8 +193,8 @@ int ldk_fp8_dequant(const uint8_t* wq, const void* scale, int dtype, void* out, 
  * wq [K, N] e4m3fn, scale [N] fp16. Replaces kernels/fp8.py:200-223 (w8a16_matmul) and its
  * kernels fp8.py:42-127, whose column masks take any N: here N % 4 == 0 (K % 8 == 0) and a
  * 16-byte aligned wq. block_n, split_k, flags and the workspace as for ldk_w4a16_matmul. More than
- * 64 rows run the prefill GEMM when N % 16 == 0 and K % 64 == 0, else the MFMA kernel in 16-row
- * blocks. */
+ * 64 rows run the prefill GEMM when K % 64 == 0 and N % 16 == 0 (with the library's choice also for
+ * other N from 1e9 multiply-adds), else the MFMA kernel in 16-row blocks. */
 int ldk_w8a16_matmul(const void* x, int64_t ldx, const uint8_t* wq, const void* scale,
                      const void* bias, void* out, int64_t ldo, int64_t M, int64_t N, int64_t K,
                      int block_n, int split_k, int flags, void* workspace, int64_t workspace_bytes,

@@ -1013,8 +1013,8 @@ extern "C" int ldk_fp8_dequant(const uint8_t* wq, const void* scale, int dtype, 
 // once per 64- or 128-row tile.
 static constexpr int64_t kW8GemmRows = 64;
 
-static bool w8_gemm_applies(int64_t M, int64_t N, int64_t K, int64_t ldx, const void* out, int64_t ldo) {
-  return ldk::gemm_supported(ldk::WFmt::kE4M3, M, N, K, 0, ldx) && ldk::aligned(out, 8) && ldo % 4 == 0;
+static bool w8_gemm_applies(int64_t M, int64_t N, int64_t K, int64_t ldx, const void* out, int64_t ldo, bool narrow = false) {
+  return ldk::gemm_supported(ldk::WFmt::kE4M3, M, N, K, 0, ldx, narrow) && ldk::aligned(out, 8) && ldo % 4 == 0;
 }
 
 // The library's choice: the GEMM for more than kW8GemmRows rows (on wide shapes more than 16)
@@ -1025,17 +1025,22 @@ static bool w8_uses_gemm(int64_t M, int64_t N, int64_t K, int64_t ldx, const voi
   // wide shapes (N >= 8192) from 17 rows: the 16-row blocks re-read all of their e4m3 weights per
   // block (gate_up M = 17 / 32 / 64: 16.9 / 20.3 / 29.7 us on the blocks, 10.9 / 11.2 / 15.5 on the
   // GEMM's 32-row tiles)
-  if (M <= (N >= 8192 ? 16 : kW8GemmRows) || block_n || split_k || (flags & (LDK_PATH_VALU | LDK_PATH_MFMA))) return false;
+  // (from 20M weights past 32 rows on narrow shapes too: M = 33 4096x14336 41 -> 29 us, 6144x4096
+  // 24 -> 16)
+  const bool large = N * K >= 20000000;
+  if (M <= (N >= 8192 ? 16 : large ? 32 : kW8GemmRows) || block_n || split_k || (flags & (LDK_PATH_VALU | LDK_PATH_MFMA))) return false;
   // narrow shapes past 64 rows keep the blocks while they fit in 256 workgroups: short K on
   // 64-column tiles (qkv M = 96 / 128: 8.1 / 8.0 us against 10.2 / 10.1 on the GEMM, o M = 160 8.3
   // against 9.7; qkv M = 160, 320 workgroups, 13.4 against 10.2), long K while they still split K
   // at least twice (down M = 96 / 128 / 160: 19.8 / 23.4 / 23.6 against 26.0 / 26.5 / 24.2; M = 192
   // in whole K 41.0 against 24.6)
-  if (N < 8192) {
+  if (N < 8192 && !large) {
     const int64_t blocks = (M + 15) / 16;
     if (w8_short_k(K) ? (N + 63) / 64 * blocks <= 256 : (N + 127) / 128 * blocks <= 128) return false;
   }
-  return w8_gemm_applies(M, N, K, ldx, out, ldo);
+  // N % 16 != 0 (the GEMM's narrow variant, dword loads) from 1e9 multiply-adds: 4120x3968, blocks
+  // against GEMM, M = 200 65 / 27 us, 3055 838 / 105; 17924x1536 M = 3055 2298 / 174
+  return w8_gemm_applies(M, N, K, ldx, out, ldo, M * N * K >= 1000000000);
 }
 
 namespace {

@@ -51,6 +51,14 @@ __device__ __forceinline__ void dma_buffer16(u32x4 rsrc, uint32_t voffset, uint3
                : "v"(voffset), "s"(rsrc), "s"(lds_base), "s"(soffset)
                : "memory");
 }
+// The same with 4 bytes per lane (lane i writes lds_base + 4 i), for rows only 4-byte aligned.
+__device__ __forceinline__ void dma_buffer4(u32x4 rsrc, uint32_t voffset, uint32_t soffset, uint32_t lds_base) {
+  uint32_t saved;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %4 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(saved)
+               : "v"(voffset), "s"(rsrc), "s"(lds_base), "s"(soffset)
+               : "memory");
+}
 // Raw buffer descriptor over [p, p + bytes): a load at an offset past it returns zeros (and, to
 // LDS, writes zeros).
 __device__ __forceinline__ u32x4 raw_rsrc(const void* p, uint32_t bytes) {

@@ -48,6 +48,7 @@ namespace {
 
 using ldk::WFmt;
 using ldk::dma_buffer16;
+using ldk::dma_buffer4;
 using ldk::lds_addr;
 using ldk::raw_rsrc;
 using ldk::ring_barrier;
@@ -103,7 +104,7 @@ struct Fmt<WFmt::kE4M3> {
   static constexpr int SZI = 0;
 };
 
-template <WFmt F, int WAVES, int MT, int S>
+template <WFmt F, int WAVES, int MT, int S, bool NARROW = false>
 struct GemmCfg {
   using T = Fmt<F>;
   static constexpr int BM = 16 * MT, NT = 4, NTHR = WAVES * 64;
@@ -112,7 +113,9 @@ struct GemmCfg {
   static constexpr int WOFF = XBYTES;                          // weights, T::WBYTES per wave
   static constexpr int SZOFF = WOFF + WAVES * T::WBYTES;       // int4 scales and zeros per wave
   static constexpr int STAGE = SZOFF + WAVES * T::SZBYTES;
-  static constexpr int LOADS = XI + T::WI + T::SZI;            // per wave and stage
+  // per wave and stage; NARROW e4m3 loads its weights 4 bytes per lane
+  static constexpr int WI = NARROW && F == WFmt::kE4M3 ? T::WBYTES / 256 : T::WI;
+  static constexpr int LOADS = XI + WI + T::SZI;
   static_assert(XI * WAVES * 8 == BM, "whole x load instructions");
   static_assert(S * STAGE <= 160 * 1024, "LDS");
 };
@@ -121,9 +124,12 @@ struct GemmCfg {
 // WAVES waves walks its half through its own ring (the second half of every stage array), and the
 // groups' accumulators meet in LDS at the end. That doubles the waves on a tile without the fp32
 // partials in memory that a split over workgroups costs.
-template <WFmt F, int WAVES, int MT, int S, int KG, bool SW>
+//
+// NARROW: N is only a multiple of 4. e4m3 K rows are then 4-byte aligned and come as dword loads to
+// LDS (four times as many), int4 scale and zero rows 8-byte aligned and come as dwords of 32 lanes.
+template <WFmt F, int WAVES, int MT, int S, int KG, bool SW, bool NARROW = false>
 __device__ __forceinline__ void gemm_body(const ldk::GemmArgs& a, int kps, float* partial, int mfast) {
-  using C = GemmCfg<F, WAVES, MT, S>;
+  using C = GemmCfg<F, WAVES, MT, S, NARROW>;
   using T = Fmt<F>;
   constexpr bool kInt4 = F == WFmt::kInt4;
   constexpr int BM = C::BM, NT = C::NT;
@@ -178,7 +184,8 @@ __device__ __forceinline__ void gemm_body(const ldk::GemmArgs& a, int kps, float
   // weights: per-lane offsets of the first K-step, plus wstep bytes per K-step (in soffset).
   // Columns are clamped so lanes past N read valid memory; their outputs are not stored.
   const u32x4 wb = raw_rsrc(a.w, (uint32_t)(kInt4 ? (int64_t)a.K / 2 * a.N : (int64_t)a.K * a.N));
-  uint32_t woff[T::WI];
+  constexpr int WI = C::WI;
+  uint32_t woff[WI];
   uint32_t wstep;
   if constexpr (kInt4) {
     // instruction sub: lane (c16, kb) takes packed row 4 sub + kb at columns n0 + 4 c16 .. + 3
@@ -186,12 +193,21 @@ __device__ __forceinline__ void gemm_body(const ldk::GemmArgs& a, int kps, float
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) woff[sub] = 4u * (uint32_t)((int64_t)(4 * sub + kb) * a.N + col);
     wstep = 32u * (uint32_t)a.N;  // 8 packed rows
+  } else if constexpr (NARROW) {
+    // instruction i fills tile rows 4 i .. + 3: lane l writes dword l % 16 of tile row 4 i + l / 16
+    const int wcol = min(n0 + 4 * (lane & 15), a.N - 4);
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+      const int tr = 4 * i + (lane >> 4), r = tr ^ ((tr >> 3) & 3);
+      woff[i] = (uint32_t)r * (uint32_t)a.N + (uint32_t)wcol;
+    }
+    wstep = 64u * (uint32_t)a.N;
   } else {
     // instruction i fills tile rows 16 i .. + 15: lane l writes tile row 16 i + l / 4, 16-byte
     // chunk l % 4, from K row (tile row) ^ ((tile row / 8) % 4) of the step
     const int wcol = min(n0 + 16 * (lane & 3), a.N - 16);
 #pragma unroll
-    for (int i = 0; i < T::WI; ++i) {
+    for (int i = 0; i < WI; ++i) {
       const int tr = 16 * i + (lane >> 2), r = tr ^ ((tr >> 3) & 3);
       woff[i] = (uint32_t)r * (uint32_t)a.N + (uint32_t)wcol;
     }
@@ -203,7 +219,7 @@ __device__ __forceinline__ void gemm_body(const ldk::GemmArgs& a, int kps, float
   const int gsh = kInt4 ? __builtin_ctz(a.group_size) - 6 : 0;  // log2(K-steps per group)
   const uint32_t szb = kInt4 ? (uint32_t)(a.K / a.group_size) * (uint32_t)a.N * 2u : 0u;
   const u32x4 sb = raw_rsrc(a.s, szb), zb = raw_rsrc(a.z, szb);
-  const uint32_t szoff = 2u * (uint32_t)(n0 + 8 * (lane & 7));
+  const uint32_t szoff = 2u * (uint32_t)(n0 + (NARROW ? 2 * (lane & 31) : 8 * (lane & 7)));
 
   auto issue = [&](unsigned char* stage, int kstep) {
     const int ks = kbeg + kstep;
@@ -211,11 +227,20 @@ __device__ __forceinline__ void gemm_body(const ldk::GemmArgs& a, int kps, float
     for (int i = 0; i < C::XI; ++i)
       dma_buffer16(xb, xoff[i], (uint32_t)(ks * kXRow), lds_addr(stage + 8 * (C::XI * wave + i) * kXRow));
 #pragma unroll
-    for (int i = 0; i < T::WI; ++i)
-      dma_buffer16(wb, woff[i], (uint32_t)ks * wstep, lds_addr(stage + C::WOFF + T::WBYTES * wave + 1024 * i));
+    for (int i = 0; i < WI; ++i) {
+      if constexpr (NARROW && !kInt4)
+        dma_buffer4(wb, woff[i], (uint32_t)ks * wstep, lds_addr(stage + C::WOFF + T::WBYTES * wave + 256 * i));
+      else
+        dma_buffer16(wb, woff[i], (uint32_t)ks * wstep, lds_addr(stage + C::WOFF + T::WBYTES * wave + 1024 * i));
+    }
     if constexpr (kInt4) {
       const uint32_t g = 2u * (uint32_t)(ks >> gsh) * (uint32_t)a.N;
-      if (lane < 8) {  // one instruction each; lanes 8-63 idle (every wave has lanes 0-7 active)
+      if constexpr (NARROW) {
+        if (lane < 32) {
+          dma_buffer4(sb, g + szoff, 0u, lds_addr(stage + C::SZOFF + 256 * wave));
+          dma_buffer4(zb, g + szoff, 0u, lds_addr(stage + C::SZOFF + 256 * wave + 128));
+        }
+      } else if (lane < 8) {  // one instruction each; lanes 8-63 idle (every wave has lanes 0-7 active)
         dma_buffer16(sb, g + szoff, 0u, lds_addr(stage + C::SZOFF + 256 * wave));
         dma_buffer16(zb, g + szoff, 0u, lds_addr(stage + C::SZOFF + 256 * wave + 128));
       }
@@ -456,6 +481,19 @@ __global__ __launch_bounds__(WAVES * KG * 64) __attribute__((amdgpu_waves_per_eu
   gemm_body<WFmt::kE4M3, WAVES, MT, S, KG, false>(a, kps, partial, mfast);
 }
 
+// The same GEMMs for N a multiple of 4 only.
+template <int WAVES, int MT, int S, int KG>
+__global__ __launch_bounds__(WAVES * KG * 64) __attribute__((amdgpu_waves_per_eu(2))) void w4a16_gemm_narrow_kernel(
+    ldk::GemmArgs a, int kps, float* partial, int mfast) {
+  gemm_body<WFmt::kInt4, WAVES, MT, S, KG, false, true>(a, kps, partial, mfast);
+}
+
+template <int WAVES, int MT, int S, int KG>
+__global__ __launch_bounds__(WAVES * KG * 64) __attribute__((amdgpu_waves_per_eu(2))) void w8a16_gemm_narrow_kernel(
+    ldk::GemmArgs a, int kps, float* partial, int mfast) {
+  gemm_body<WFmt::kE4M3, WAVES, MT, S, KG, false, true>(a, kps, partial, mfast);
+}
+
 // The same GEMMs with SwiGLU in the epilogue (GemmArgs::swiglu; no K split).
 template <int WAVES, int MT, int S, int KG>
 __global__ __launch_bounds__(WAVES * KG * 64) __attribute__((amdgpu_waves_per_eu(2))) void w4a16_gemm_swiglu_kernel(
@@ -545,8 +583,13 @@ GemmShape pick_shape(WFmt f, int64_t M, int64_t N, int64_t K, int block_n, int s
     if (!long_k) return 1;
     const int64_t most = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(6, steps / 8), room));
     int64_t best = 1;
-    for (int64_t sp = 2; sp <= most; ++sp)  // ceil(t sp / 256) / sp < ceil(t best / 256) / best
-      if (((t * sp + 255) / 256) * best < ((t * best + 255) / 256) * sp) best = sp;
+    for (int64_t sp = 2; sp <= most; ++sp) {  // ceil(t sp / 256) / sp < ceil(t best / 256) / best
+      const int64_t a = ((t * sp + 255) / 256) * best, b = ((t * best + 255) / 256) * sp;
+      // equal shares of a K of 192 steps or more: the larger count, up to two workgroups per CU,
+      // which hide each other's waits (4096x14336 M = 777: 4 splits instead of 2, e4m3 122 -> 110 us,
+      // int4 135 -> 112; M = 1500: 2 instead of 1, 217 -> 190 and 244 -> 204; 1536x8960, 140 steps, M = 1500 61 against 63)
+      if (a < b || (a == b && steps >= 192 && t * sp <= 512)) best = sp;
+    }
     return (int)best;
   };
   // long K with at least 16 row tiles: row tiles on the grid's fast axis (down M = 1024 / 2048:
@@ -609,10 +652,18 @@ int launch(const ldk::GemmArgs& a, int splits, int mfast, hipStream_t s) {
     }
   }
   if (a.swiglu) return ldk::fail(LDK_ERR_UNSUPPORTED, "gemm: SwiGLU epilogue not built for %d x %d tiles", WAVES, MT);
-  if constexpr (F == WFmt::kInt4)
-    w4a16_gemm_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
-  else
-    w8a16_gemm_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
+  const bool narrow = a.N % (F == WFmt::kInt4 ? 8 : 16) != 0;
+  if constexpr (F == WFmt::kInt4) {
+    if (narrow)
+      w4a16_gemm_narrow_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
+    else
+      w4a16_gemm_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
+  } else {
+    if (narrow)
+      w8a16_gemm_narrow_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
+    else
+      w8a16_gemm_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
+  }
   int st = ldk::check_launch(F == WFmt::kInt4 ? "w4a16_gemm" : "w8a16_gemm");
   if (st || nz == 1) return st;
   const int64_t quads = (int64_t)a.M * (a.N / 4);
@@ -646,13 +697,13 @@ int launch_fmt(const ldk::GemmArgs& a, hipStream_t s) {
 
 namespace ldk {
 
-bool gemm_supported(WFmt f, int64_t M, int64_t N, int64_t K, int group_size, int64_t ldx) {
+bool gemm_supported(WFmt f, int64_t M, int64_t N, int64_t K, int group_size, int64_t ldx, bool narrow) {
   if (M <= 0 || N <= 0 || K <= 0 || K % kStep) return false;
   if (f == WFmt::kInt4) {
-    if (group_size < kStep || (group_size & (group_size - 1)) || K % group_size || N % 8) return false;
+    if (group_size < kStep || (group_size & (group_size - 1)) || K % group_size || N % (narrow ? 4 : 8)) return false;
     // scales and zeros are read through 32-bit buffer offsets
     if ((K / group_size) * N * 2 >= (int64_t(1) << 31)) return false;
-  } else if (N % 16) {
+  } else if (N % (narrow ? 4 : 16)) {
     return false;
   }
   if ((M + 63) / 64 > 65535 || (M * (N / 4) + 255) / 256 > INT32_MAX) return false;
@@ -665,7 +716,7 @@ bool gemm_supported(WFmt f, int64_t M, int64_t N, int64_t K, int group_size, int
 
 int gemm_launch(WFmt f, const GemmArgs& a, hipStream_t s) {
   const char* fn = f == WFmt::kInt4 ? "w4a16_gemm" : "w8a16_gemm";
-  if (!gemm_supported(f, a.M, a.N, a.K, a.group_size, a.ldx))
+  if (!gemm_supported(f, a.M, a.N, a.K, a.group_size, a.ldx, true))
     return fail(LDK_ERR_UNSUPPORTED, "%s: shape M=%d N=%d K=%d group_size=%d not supported", fn, a.M, a.N, a.K,
                 a.group_size);
   if (a.swiglu && !gemm_swiglu_applies(f, a.M, a.N, a.K, a.group_size, a.ldx, a.block_n, a.split_k,

@@ -405,3 +405,23 @@ def test_decode_rows_on_large_weights(M, N, K):
     y = w8a16_matmul(x, wq, s, bias=b).double()
     ref = x.double() @ (wq.float().double() * s.double()).contiguous() + b.double()
     assert (y - ref).abs().max() <= 2e-2 and (y - ref).norm() / ref.norm() <= 1e-3
+
+
+@pytest.mark.parametrize("M,N,K", [(1030, 1012, 2048), (400, 4120, 1280), (130, 17924, 1024), (2100, 268, 4096),
+                                   (777, 516, 9984), (33, 6140, 12288)])
+def test_prefill_gemm_narrow_rows(M, N, K):
+    """Prefill rows with N % 16 != 0 from 1e9 multiply-adds: the prefill GEMM on dword loads, over its
+    tile shapes (one and two K groups, 1 to 4 column groups, split K), with partial row and column
+    tiles. Against float64 on the GPU at the suite's matmul bounds; a GEMM that the caller forces
+    still refuses these N."""
+    assert config_for(M, N, K).startswith("gemm,")
+    with pytest.raises(RuntimeError):
+        config_for(M, N, K, {"prefill": "gemm"})
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.02).half()
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    b = torch.randn(N, generator=g, device="cuda").half()
+    wq, s = quantize_fp8(w)
+    y = w8a16_matmul(x, wq, s, bias=b).double()
+    ref = x.double() @ (wq.float().double() * s.double()).contiguous() + b.double()
+    assert (y - ref).abs().max() <= 2e-2 and (y - ref).norm() / ref.norm() <= 1e-3

@@ -679,3 +679,24 @@ def test_decode_rows_on_large_weights(M, N, K, plan):
     ref = x.double() @ w
     # the dequantized weight is rounded to fp16 nowhere in the factored form: fp32 sums, one rounding
     assert (y - ref).norm() / ref.norm() <= 1e-3 and ((y - ref).abs() / ref.abs().clamp_min(1.0)).max() <= 5e-3
+
+
+@pytest.mark.parametrize("M,N,K", [(1030, 1012, 2048), (400, 4124, 1280), (130, 17924, 1024), (2100, 268, 4096),
+                                   (777, 516, 9984), (260, 6140, 12288)])
+def test_prefill_gemm_narrow_rows(M, N, K):
+    """Prefill rows with N % 8 == 4 from 1e9 multiply-adds: the prefill GEMM with its scales and zeros
+    in dword loads, over its tile shapes, with partial row and column tiles; float64 on the GPU from
+    the weights as dequantize_ref rounds them. A GEMM that the caller forces still refuses these N."""
+    assert config_for(M, N, K).startswith("gemm,")
+    with pytest.raises(RuntimeError):
+        config_for(M, N, K, config={"prefill": "gemm"})
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    q = torch.randint(0, 16, (K, N), generator=g, device="cuda").int()
+    s = (torch.rand(K // 128, N, generator=g, device="cuda") * 0.004 + 0.002).half()
+    z = torch.randint(6, 10, (K // 128, N), generator=g, device="cuda").half()
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    b = torch.randn(N, generator=g, device="cuda").half()
+    y = w4a16_matmul(x, pack_int4(q), s, z, bias=b).double()
+    w = ((q.half().view(K // 128, 128, N) - z[:, None]) * s[:, None]).view(K, N)
+    ref = x.double() @ w.double() + b.double()
+    assert (y - ref).norm() / ref.norm() <= 1e-3 and ((y - ref).abs() / ref.abs().clamp_min(1.0)).max() <= 5e-3
