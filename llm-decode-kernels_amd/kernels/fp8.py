@@ -120,19 +120,21 @@ def w8a16_matmul(x, wq, scale, bias=None, config=None):
     dev = _lib.require_gpu(x, wq, scale, bias, what="w8a16_matmul")
     if x.dtype != torch.float16 or scale.dtype != torch.float16:
         raise ValueError("w8a16_matmul: x and scale must be float16")
-    x2 = x.reshape(-1, K)
+    flat = x.dim() == 2
+    x2 = x if flat else x.reshape(-1, K)
     if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
     M = x2.shape[0]
     q = wq if wq.is_contiguous() else wq.contiguous()
     s = scale.contiguous()
     b = None if bias is None else bias.to(torch.float16).contiguous()
-    block_n, split_k, flags = _tuning(config, M, N, K)
+    block_n, split_k, flags = _tuning(config, M, N, K) if config else (0, 0, 0)
     out = torch.empty((M, N), dtype=torch.float16, device=dev)
     with _lib.device_guard(dev):
         ws, ws_bytes = _lib.workspace(dev)
+        # the tensors are this frame's locals, so plain addresses outlive the call
         st = _lib.load().ldk_w8a16_matmul(
-            _lib.ptr(x2), x2.stride(0), _lib.ptr(q), _lib.ptr(s), _lib.ptr(b), _lib.ptr(out),
-            out.stride(0), M, N, K, block_n, split_k, flags, ws, ws_bytes, _lib.stream(dev))
+            x2.data_ptr(), x2.stride(0), q.data_ptr(), s.data_ptr(), None if b is None else b.data_ptr(),
+            out.data_ptr(), N, M, N, K, block_n, split_k, flags, ws, ws_bytes, _lib.stream(dev))
     _lib.check(st, "w8a16_matmul")
-    return out.view(*x.shape[:-1], N)
+    return out if flat else out.view(*x.shape[:-1], N)

@@ -19,7 +19,8 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, residual=N
     (rmsnorm.py:44-68)."""
     shape = x.shape
     N = shape[-1]
-    x2 = x.reshape(-1, N)
+    flat = x.dim() == 2
+    x2 = x if flat else x.reshape(-1, N)
     assert x2.stride(-1) == 1 and weight.is_contiguous()
     dev = _lib.require_gpu(x, weight, residual, what="rmsnorm")
     if x.dtype != torch.float16 or weight.dtype != torch.float16:
@@ -28,19 +29,24 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, residual=N
     out = torch.empty((M, N), dtype=x.dtype, device=dev)
     r2 = res_out = None
     if residual is not None:
-        r2 = residual.reshape(-1, N)
+        r2 = residual if residual.shape == x2.shape else residual.reshape(-1, N)
         if r2.stride(-1) != 1:
             r2 = r2.contiguous()
         res_out = torch.empty_like(out)
     with _lib.device_guard(dev):
+        # the tensors are this frame's locals, so plain addresses outlive the call
+        if r2 is None:
+            res = (None, 0, None, 0)
+        else:
+            res = (r2.data_ptr(), r2.stride(0), res_out.data_ptr(), N)
         st = _lib.load().ldk_rmsnorm(
-            _lib.ptr(x2), x2.stride(0), _lib.ptr(r2), 0 if r2 is None else r2.stride(0),
-            _lib.ptr(weight), _lib.ptr(out), out.stride(0), _lib.ptr(res_out),
-            0 if res_out is None else res_out.stride(0), M, N, float(eps), _lib.stream(dev))
+            x2.data_ptr(), x2.stride(0), res[0], res[1], weight.data_ptr(), out.data_ptr(), N, res[2],
+            res[3], M, N, float(eps), _lib.stream(dev))
     _lib.check(st, "rmsnorm")
-    if residual is None:
-        return out.view(shape)
-    return out.view(shape), res_out.view(shape)
+    if not flat:
+        out = out.view(shape)
+        res_out = None if res_out is None else res_out.view(shape)
+    return out if residual is None else (out, res_out)
 
 
 def rmsnorm_bytes(M: int, N: int, residual: bool, elem: int = 2) -> int:

@@ -106,10 +106,11 @@ def _decode(x2, qweight, scales, zeros, bias, group_size, block_n, split_k, flag
     dev = x2.device
     with _lib.device_guard(dev):
         ws, ws_bytes = _lib.workspace(dev)
+        # the tensors are this frame's and the caller's locals, so plain addresses outlive the call
         st = _lib.load().ldk_w4a16_matmul(
-            _lib.ptr(x2), x2.stride(0), _lib.ptr(qweight), _lib.ptr(scales), _lib.ptr(zeros),
-            _lib.ptr(bias), _lib.ptr(out), out.stride(0), M, N, K, group_size, block_n, split_k,
-            flags, ws, ws_bytes, _lib.stream(dev))
+            x2.data_ptr(), x2.stride(0), qweight.data_ptr(), scales.data_ptr(), zeros.data_ptr(),
+            None if bias is None else bias.data_ptr(), out.data_ptr(), N, M, N, K, group_size,
+            block_n, split_k, flags, ws, ws_bytes, _lib.stream(dev))
     _lib.check(st, "w4a16_matmul")
     return out
 
@@ -122,7 +123,8 @@ def w4a16_matmul(x, qweight, scales, zeros, group_size=128, bias=None, config=No
     dev = _lib.require_gpu(x, qweight, scales, zeros, bias, what="w4a16_matmul")
     if x.dtype != torch.float16 or scales.dtype != torch.float16 or zeros.dtype != torch.float16:
         raise ValueError("w4a16_matmul: x, scales and zeros must be float16")
-    x2 = x.reshape(-1, K)
+    flat = x.dim() == 2
+    x2 = x if flat else x.reshape(-1, K)
     if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
     M = x2.shape[0]
@@ -130,15 +132,16 @@ def w4a16_matmul(x, qweight, scales, zeros, group_size=128, bias=None, config=No
     s = scales if scales.is_contiguous() else scales.contiguous()
     z = zeros if zeros.is_contiguous() else zeros.contiguous()
     b = None if bias is None else bias.to(torch.float16).contiguous()
-    block_n, split_k, flags = _tuning(config, M, N, K, group_size)
+    block_n, split_k, flags = _tuning(config, M, N, K, group_size) if config else (0, 0, 0)
     out = torch.empty((M, N), dtype=torch.float16, device=dev)
     _decode(x2, qw, s, z, b, group_size, block_n, split_k, flags, out)
     # the library's choice is recorded for the decode shapes it chose (w4a16.py:322-326): a call
     # whose config forced a variant records nothing, as the reference's forced path picks nothing
-    key = (min(_next_pow2(M), 16), N, K, bias is not None)
-    if M <= 16 and not config and key not in _decode_choice:
-        _decode_choice[key] = config_for(M, N, K, group_size)
-    return out.view(*x.shape[:-1], N)
+    if M <= 16 and not config:
+        key = (min(_next_pow2(M), 16), N, K, bias is not None)
+        if key not in _decode_choice:
+            _decode_choice[key] = config_for(M, N, K, group_size)
+    return out if flat else out.view(*x.shape[:-1], N)
 
 
 def config_for(M: int, N: int, K: int, group_size: int = 128, config: dict | None = None) -> str:
