@@ -170,7 +170,8 @@ def prefill_supported(head_dim: int, max_len: int, batch: int, tokens: int) -> b
             and batch == 1 and 1 <= tokens <= 1 << 24)
 
 
-# Most position ranges the o projection's merge takes (csrc/w4a16.hip, kAttnRanges).
+# Most position ranges the o projection's merge takes (csrc/w4a16.hip, kAttnRanges); the runner takes
+# decode_attention and its own merge launch on caches longer than QwenRunner.merge_max_len.
 MERGE_MAX_RANGES = 4
 # Most byte ranges one launch warms (csrc/warm.h, kWarmMax).
 WARM_MAX_RANGES = _lib.WARM_MAX_RANGES

@@ -9,7 +9,8 @@ launch. The staged activations follow the standalone kernels' rounding steps (`k
 `kernels.swiglu`); SwiGLU's are bit-identical to them, RMSNorm's can differ from them by one fp16
 ulp, because the row's sum of squares is reduced in another order.
 
-Rows other than one (prefill) and group sizes other than 128 run the two ops back to back.
+Rows other than one (prefill), group sizes other than 128 and projections past FUSED_NORM_MAX_N or
+FUSED_MAX_WEIGHTS run the two ops back to back.
 """
 
 from __future__ import annotations
