@@ -74,12 +74,18 @@ __device__ __forceinline__ uint16_t from_f32<uint16_t>(float v) {
 // 1293 us on 14336 x 4096 fp16; this 59 us, of which the first launch is about 20.
 __device__ __forceinline__ float fp8_scale(float amax) { return fmaxf(amax / 448.0f, 1e-12f); }
 
-// V elements of T per load (1: any base and K).
+// V elements of T per load (1: any base and K). A launch holds fewer than 2^32 threads per grid
+// dimension, so channels past kAbsmaxBlocks go to the grid's second dimension.
+constexpr int64_t kAbsmaxBlocks = 1 << 20;
+
 template <typename T, int V>
-__global__ __launch_bounds__(256) void fp8_absmax_kernel(const T* __restrict__ w, T* __restrict__ amax_out, int64_t K) {
+__global__ __launch_bounds__(256) void fp8_absmax_kernel(const T* __restrict__ w, T* __restrict__ amax_out, int64_t N,
+                                                         int64_t K) {
   typedef T tv_t __attribute__((ext_vector_type(V)));
   __shared__ float part[4];
-  const T* row = w + (int64_t)blockIdx.x * K;
+  const int64_t n = (int64_t)blockIdx.y * kAbsmaxBlocks + blockIdx.x;
+  if (n >= N) return;  // uniform
+  const T* row = w + n * K;
   float amax = 0.0f;
   for (int64_t k = threadIdx.x * V; k < K; k += 256 * V) {
     const tv_t v = *reinterpret_cast<const tv_t*>(row + k);
@@ -90,7 +96,7 @@ __global__ __launch_bounds__(256) void fp8_absmax_kernel(const T* __restrict__ w
   for (int o = 1; o < 64; o *= 2) amax = fmaxf(amax, __shfl_xor(amax, o));
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;
   __syncthreads();
-  if (threadIdx.x == 0) amax_out[blockIdx.x] = from_f32<T>(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
+  if (threadIdx.x == 0) amax_out[n] = from_f32<T>(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
 }
 
 template <typename T>
@@ -945,11 +951,12 @@ int launch_fp8_quantize(const T* w, uint8_t* wq, T* scale, int64_t N, int64_t K,
   const int64_t tiles = ((N + kFCols - 1) / kFCols) * ((K + kFRows - 1) / kFRows);
   if (tiles > INT32_MAX || N > INT32_MAX) return ldk::fail(LDK_ERR_UNSUPPORTED, "fp8_quantize: too large");
   const bool vec = K % 8 == 0 && ldk::aligned(w, 16), quad = N % 4 == 0 && ldk::aligned(wq, 4);
+  const dim3 rows((unsigned)std::min(N, kAbsmaxBlocks), (unsigned)((N + kAbsmaxBlocks - 1) / kAbsmaxBlocks));
   (void)hipGetLastError();
   if (vec)
-    fp8_absmax_kernel<T, 8><<<(unsigned)N, 256, 0, s>>>(w, scale, K);
+    fp8_absmax_kernel<T, 8><<<rows, 256, 0, s>>>(w, scale, N, K);
   else
-    fp8_absmax_kernel<T, 1><<<(unsigned)N, 256, 0, s>>>(w, scale, K);
+    fp8_absmax_kernel<T, 1><<<rows, 256, 0, s>>>(w, scale, N, K);
   auto tile = [&](auto kernel) { kernel<<<(unsigned)tiles, 256, 0, s>>>(w, scale, wq, N, K); };
   if (vec && quad)
     tile(fp8_quantize_kernel<T, 8, 4>);

@@ -216,3 +216,18 @@ def test_fp8_convert_tiles(N, K):
     owq, os_ = of.quantize_fp8(w32.numpy())
     assert np.array_equal(wq.view(torch.uint8).cpu().numpy(), owq) and np.array_equal(to_np(s), os_)
     assert np.array_equal(to_np(dequantize_fp8(wq, s)), of.dequantize_fp8(owq, os_))
+
+
+@pytest.mark.parametrize("N", [(1 << 20) + 1, (1 << 24) + 133])
+def test_fp8_quantize_many_channels(N):
+    """More channels than the absmax launch has workgroups, and than it could have at one each."""
+    from kernels.fp8 import quantize_fp8
+    from oracle import fp8 as of
+
+    g = torch.Generator(device="cuda").manual_seed(N)
+    w = (torch.randn(N, 8, generator=g, device="cuda") * torch.rand(N, 1, generator=g, device="cuda")).half()
+    wq, s = quantize_fp8(w)
+    rows = torch.cat([torch.arange(300), torch.arange((1 << 20) - 150, (1 << 20) + 1), torch.arange(N - 300, N)])
+    owq, os_ = of.quantize_fp8(w[rows].cpu().numpy())
+    assert np.array_equal(bits16(s[rows]), bits16(os_))
+    assert np.array_equal(to_np(wq.view(torch.uint8)[:, rows]), owq.view(np.uint8))
