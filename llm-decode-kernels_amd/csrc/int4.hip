@@ -280,13 +280,14 @@ int log2_exact(int64_t v) {
   return s;
 }
 
-// Launches the tiled quantizer for group sizes 32 .. 512 (powers of two) and 16-byte aligned weights,
-// else the one-thread-per-group one.
+// Launches the tiled quantizer for group sizes 32 .. 512 (powers of two), 16-byte aligned weights and
+// fewer than 2^24 tiles (a launch holds fewer than 2^32 threads per grid dimension), else the
+// one-thread-per-group one.
 template <typename T>
 void launch_quantize(const T* w, uint32_t* qweight, T* scales, T* zeros, int64_t N, int64_t K, int G, hipStream_t s) {
   const int64_t tiles = (K / G) * ((N + kQCols - 1) / kQCols);
   auto tiled = [&](auto kernel) { kernel<<<(unsigned)tiles, 256, 0, s>>>(w, qweight, scales, zeros, N, K); };
-  if (ldk::aligned(w, 16) && tiles <= INT32_MAX) {
+  if (ldk::aligned(w, 16) && tiles < (int64_t(1) << 24)) {
     switch (G) {
       case 32: return tiled(quantize_rtn_tile_kernel<T, 4>);
       case 64: return tiled(quantize_rtn_tile_kernel<T, 8>);
