@@ -29,16 +29,6 @@ __device__ __forceinline__ uint32_t e4m3_encode2(float a, float b) {
   return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false) & 0xffffu;
 }
 
-// e4m3fn byte -> float, written from the format (used where bit-exactness is the contract).
-__device__ __forceinline__ float e4m3_decode(uint32_t b) {
-  const uint32_t e = (b >> 3) & 0xFu, m = b & 7u;
-  float v;
-  if (e == 0) v = (float)m * 0.001953125f;  // m * 2^-9
-  else if (e == 15 && m == 7) v = __builtin_nanf("");
-  else v = __builtin_bit_cast(float, ((e + 120u) << 23) | (m << 20));
-  return (b & 0x80u) ? -v : v;
-}
-
 template <typename T>
 __device__ __forceinline__ float to_f32(T v);
 template <>
@@ -67,11 +57,13 @@ __device__ __forceinline__ uint16_t from_f32<uint16_t>(float v) {
 //  1. fp8_absmax_kernel, one workgroup per channel: absmax of its row, left in scale[n] (the largest
 //     of T's values is one of T's values, so nothing is lost there);
 //  2. fp8_quantize_kernel, tiles of 128 channels x 64 k turned through LDS: rows are read in
-//     128-byte runs and wq is written in 128-byte runs of one k row;
+//     128-byte runs and wq is written in 128-byte runs of one k row, 4 codes a store at any
+//     alignment (a byte a store took 58 against 51 us at 14333 x 4096, 22.7 against 20.2 at
+//     1533 x 8960);
 //  3. fp8_scale_kernel: scale[n] = the rounded fp32 scale.
 // Arithmetic as fp8.py:27-29 in float32: scale = max(absmax / 448, 1e-12);
 // wq = e4m3(clamp(w / scale, -448, 448)). One thread per channel, reading its row twice, took
-// 1293 us on 14336 x 4096 fp16; this 59 us, of which the first launch is about 20.
+// 1293 us on 14336 x 4096 fp16; this 54 us a call, of which the first launch is about 20.
 __device__ __forceinline__ float fp8_scale(float amax) { return fmaxf(amax / 448.0f, 1e-12f); }
 
 // V elements of T per load (1: any base and K). A launch holds fewer than 2^32 threads per grid
@@ -106,10 +98,13 @@ __global__ __launch_bounds__(256) void fp8_scale_kernel(T* __restrict__ scale, i
 }
 
 constexpr int kFCols = 128, kFRows = 64;  // channels and k of a tile
+// Four codes of a k row, at any address (N odd: no k row is aligned); a global access of 4 bytes
+// needs no alignment on this chip.
+typedef uint32_t bytes4_t __attribute__((aligned(1)));
 
-// V: elements of T per load of w (8, or 1 for any base and K); S: bytes per store of wq (4 where the
-// k rows are 4-byte aligned, else 1).
-template <typename T, int V, int S>
+// V: elements of T per load of w (8, or 1 for any base and K). TAIL: N is no multiple of 4, so a k row's
+// last codes are stored one by one.
+template <typename T, int V, bool TAIL>
 __global__ __launch_bounds__(256) void fp8_quantize_kernel(const T* __restrict__ w, const T* __restrict__ amax,
                                                            uint8_t* __restrict__ wq, int64_t N, int64_t K) {
   typedef T tv_t __attribute__((ext_vector_type(V)));
@@ -159,14 +154,15 @@ __global__ __launch_bounds__(256) void fp8_quantize_kernel(const T* __restrict__
     }
   }
   __syncthreads();
-  const int nn = tid * S % kFCols;
-  for (int r = tid * S / kFCols; r < kFRows; r += 256 * S / kFCols) {
-    if (k0 + r >= K || n0 + nn >= N) continue;
+  const int nn = tid * 4 % kFCols;
+  const int64_t left = N - n0 - nn;  // channels from this thread's first on
+  if (left <= 0) return;
+  for (int r = tid * 4 / kFCols; r < kFRows && k0 + r < K; r += 256 * 4 / kFCols) {
     uint8_t* dst = wq + (k0 + r) * N + n0 + nn;
-    if constexpr (S == 4)
-      *reinterpret_cast<uint32_t*>(dst) = *reinterpret_cast<const uint32_t*>(&tile[r][nn]);
+    if (!TAIL || left >= 4)
+      *reinterpret_cast<bytes4_t*>(dst) = *reinterpret_cast<const uint32_t*>(&tile[r][nn]);
     else
-      *dst = tile[r][nn];
+      for (int j = 0; j < left; ++j) dst[j] = tile[r][nn + j];
   }
 }
 
@@ -174,9 +170,11 @@ __global__ __launch_bounds__(256) void fp8_quantize_kernel(const T* __restrict__
 // product of an e4m3 value and an fp16/bf16 scale is exact in fp32). Tiles of 64 channels x 64 k
 // turned through LDS: a thread decodes 4 channels x 4 k and leaves each channel's 4 values as one
 // LDS write; an output row leaves in 16-byte stores (VS; one value each where the rows are not
-// 16-byte aligned). L: bytes per load (4 where the k rows are 4-byte aligned, else 1). One thread
-// per output, each reading a byte of its own line, took 236 us on 14336 x 4096 fp16 and 68 on
-// 1533 x 8960 bf16; this 47 and 17 (byte loads: the 4-byte ones need N % 4 == 0).
+// 16-byte aligned). L: bytes per load (4 at any address, 1 for N < 4). Bound by the vector
+// instructions per value next to memory, so the codes go through v_cvt_pk_f32_fp8, two at a time:
+// decoded in software, with byte loads where the k rows are not 4-byte aligned, 14336 x 4096 fp16 took
+// 34.8 us a call, 14333 x 4096 39.9 and 1533 x 8960 bf16 14.9; this 27.7, 27.9 and 10.4 (one thread
+// per output, each reading a byte of its own line, 236 us and 66 for the first and the last).
 template <typename T, int L, bool VS>
 __global__ __launch_bounds__(256) void fp8_dequant_kernel(const uint8_t* __restrict__ wq, const T* __restrict__ scale,
                                                           T* __restrict__ out, int64_t N, int64_t K) {
@@ -186,32 +184,50 @@ __global__ __launch_bounds__(256) void fp8_dequant_kernel(const uint8_t* __restr
   const int64_t kt = (K + C - 1) / C;
   const int64_t k0 = blockIdx.x % kt * C, n0 = blockIdx.x / kt * C;
   const int tid = threadIdx.x, c = tid % 16 * 4, kr = tid / 16 * 4;
+  // L == 4: a word that would pass its row's end starts at N - 4 and is shifted
+  const int64_t at = min(n0 + c, N - 4);
+  const uint32_t past = min((uint32_t)(n0 + c - at), 3u) * 8u;
   uint32_t word[4];  // row kr + i: the bytes of channels c .. c + 3 (clamped ones are not stored)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint8_t* src = wq + min(k0 + kr + i, K - 1) * N;
-    if constexpr (L == 4) {  // N % 4 == 0
-      word[i] = *reinterpret_cast<const uint32_t*>(src + min(n0 + c, N - 4));
+    if constexpr (L == 4) {
+      word[i] = *reinterpret_cast<const bytes4_t*>(src + at) >> past;
     } else {
       word[i] = 0;
 #pragma unroll
       for (int j = 0; j < 4; ++j) word[i] |= (uint32_t)src[min(n0 + c + j, N - 1)] << (8 * j);
     }
   }
+  uint32_t nan_codes = 0;  // bit 7 of a byte: one of the words holds 0x7F or 0xFF there
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float sc = to_f32<T>(scale[min(n0 + c + j, N - 1)]);
-    t4_t v;
+  for (int i = 0; i < 4; ++i) nan_codes |= (word[i] & 0x7F7F7F7Fu) + 0x01010101u;
+  const bool nans = __any((nan_codes & 0x80808080u) != 0);
+  float sc[4];
+  t4_t v[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float p = e4m3_decode((word[i] >> (8 * j)) & 0xFFu) * sc;
+  for (int j = 0; j < 4; ++j) sc[j] = to_f32<T>(scale[min(n0 + c + j, N - 1)]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float2_t lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)word[i], false);
+    const float2_t hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)word[i], true);
+    float w[4] = {lo[0], lo[1], hi[0], hi[1]};
+    if (nans) {  // the instruction turns 0x7F into a NaN with the sign bit set
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (((word[i] >> (8 * j)) & 0xFFu) == 0x7Fu) w[j] = __builtin_nanf("");
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float p = w[j] * sc[j];
       // Keep the f32 product: fused into one v_fma_mix with a +0 addend, the fp16 conversion would
       // turn a -0 product (code 0x80) into +0.
       asm volatile("" : "+v"(p));
-      v[i] = from_f32<T>(p);
+      v[j][i] = from_f32<T>(p);
     }
-    *reinterpret_cast<t4_t*>(&tile[c + j][kr]) = v;
   }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) *reinterpret_cast<t4_t*>(&tile[c + j][kr]) = v[j];
   __syncthreads();
   if constexpr (VS) {
     typedef T tv_t __attribute__((ext_vector_type(E)));
@@ -950,7 +966,7 @@ template <typename T>
 int launch_fp8_quantize(const T* w, uint8_t* wq, T* scale, int64_t N, int64_t K, hipStream_t s) {
   const int64_t tiles = ((N + kFCols - 1) / kFCols) * ((K + kFRows - 1) / kFRows);
   if (tiles > INT32_MAX || N > INT32_MAX) return ldk::fail(LDK_ERR_UNSUPPORTED, "fp8_quantize: too large");
-  const bool vec = K % 8 == 0 && ldk::aligned(w, 16), quad = N % 4 == 0 && ldk::aligned(wq, 4);
+  const bool vec = K % 8 == 0 && ldk::aligned(w, 16);
   const dim3 rows((unsigned)std::min(N, kAbsmaxBlocks), (unsigned)((N + kAbsmaxBlocks - 1) / kAbsmaxBlocks));
   (void)hipGetLastError();
   if (vec)
@@ -958,14 +974,14 @@ int launch_fp8_quantize(const T* w, uint8_t* wq, T* scale, int64_t N, int64_t K,
   else
     fp8_absmax_kernel<T, 1><<<rows, 256, 0, s>>>(w, scale, N, K);
   auto tile = [&](auto kernel) { kernel<<<(unsigned)tiles, 256, 0, s>>>(w, scale, wq, N, K); };
-  if (vec && quad)
-    tile(fp8_quantize_kernel<T, 8, 4>);
+  if (vec && N % 4 == 0)
+    tile(fp8_quantize_kernel<T, 8, false>);
   else if (vec)
-    tile(fp8_quantize_kernel<T, 8, 1>);
-  else if (quad)
-    tile(fp8_quantize_kernel<T, 1, 4>);
+    tile(fp8_quantize_kernel<T, 8, true>);
+  else if (N % 4 == 0)
+    tile(fp8_quantize_kernel<T, 1, false>);
   else
-    tile(fp8_quantize_kernel<T, 1, 1>);
+    tile(fp8_quantize_kernel<T, 1, true>);
   fp8_scale_kernel<T><<<blocks_for(N, 256), 256, 0, s>>>(scale, N);
   return ldk::check_launch("fp8_quantize");
 }
@@ -974,13 +990,12 @@ template <typename T>
 int launch_fp8_dequant(const uint8_t* wq, const T* scale, T* out, int64_t N, int64_t K, hipStream_t s) {
   const int64_t tiles = ((N + 63) / 64) * ((K + 63) / 64);
   if (tiles > INT32_MAX) return ldk::fail(LDK_ERR_UNSUPPORTED, "fp8_dequant: too large");
-  const bool quad = N % 4 == 0 && ldk::aligned(wq, 4);
   const bool vec = K * (int64_t)sizeof(T) % 16 == 0 && ldk::aligned(out, 16);
   (void)hipGetLastError();
   auto tile = [&](auto kernel) { kernel<<<(unsigned)tiles, 256, 0, s>>>(wq, scale, out, N, K); };
-  if (quad && vec)
+  if (N >= 4 && vec)
     tile(fp8_dequant_kernel<T, 4, true>);
-  else if (quad)
+  else if (N >= 4)
     tile(fp8_dequant_kernel<T, 4, false>);
   else if (vec)
     tile(fp8_dequant_kernel<T, 1, true>);

@@ -231,3 +231,23 @@ def test_fp8_quantize_many_channels(N):
     owq, os_ = of.quantize_fp8(w[rows].cpu().numpy())
     assert np.array_equal(bits16(s[rows]), bits16(os_))
     assert np.array_equal(to_np(wq.view(torch.uint8)[:, rows]), owq.view(np.uint8))
+
+
+@pytest.mark.parametrize("N", [1, 5, 64])
+def test_fp8_dequantize_every_code(N):
+    """The conversion instruction against the format's table: every code times scales of both signs,
+    to zero, to fp16's subnormals and past its range."""
+    from kernels.fp8 import FP8, dequantize_fp8
+    from oracle import fp8 as of
+
+    codes = np.repeat(np.arange(256, dtype=np.uint8)[:, None], N, 1)
+    scales = np.resize(np.array([1.0, -0.37, 6e-8, 146.0, -3e-5, 0.0, -0.0, 1e-3], dtype=np.float32), N)
+    nan = (np.arange(256) & 0x7F) == 0x7F
+    for dt in (np.float32, np.float16):
+        s = scales.astype(dt)
+        got = to_np(dequantize_fp8(dev(codes).view(FP8), dev(s)))
+        with np.errstate(over="ignore", invalid="ignore"):
+            ref = (of.e4m3_decode(codes) * s.astype(np.float32)).astype(dt).T
+        assert np.isnan(got[:, nan]).all() and np.array_equal(np.signbit(got[:, nan]), codes.T[:, nan] > 127)
+        bits = [np.ascontiguousarray(a[:, ~nan]).view(np.uint8) for a in (got, ref)]
+        assert np.array_equal(*bits)
