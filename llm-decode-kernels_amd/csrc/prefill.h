@@ -41,7 +41,7 @@ struct GemmArgs {
 // multiple of 8; kE4M3: N a multiple of 16; sizes within its 32-bit buffer offsets), and launches
 // it (with a K split over workgroups when the shape's K is long and the workspace holds the
 // partials; a second launch then sums them in split order). Both leave the last-error message on
-// failure. With `narrow`, also N a multiple of 4 only (gemm_launch takes those too).
+// failure. With `narrow`, kE4M3 also takes N a multiple of 4 only (gemm_launch takes those too).
 bool gemm_supported(WFmt f, int64_t M, int64_t N, int64_t K, int group_size, int64_t ldx, bool narrow = false);
 int gemm_launch(WFmt f, const GemmArgs& a, hipStream_t stream);
 

@@ -113,8 +113,9 @@ struct GemmCfg {
   static constexpr int WOFF = XBYTES;                          // weights, T::WBYTES per wave
   static constexpr int SZOFF = WOFF + WAVES * T::WBYTES;       // int4 scales and zeros per wave
   static constexpr int STAGE = SZOFF + WAVES * T::SZBYTES;
-  // per wave and stage; NARROW e4m3 loads its weights 4 bytes per lane
-  static constexpr int WI = NARROW && F == WFmt::kE4M3 ? T::WBYTES / 256 : T::WI;
+  static_assert(!NARROW || F == WFmt::kE4M3, "int4 columns come in eights");
+  // per wave and stage; NARROW loads its weights 4 bytes per lane
+  static constexpr int WI = NARROW ? T::WBYTES / 256 : T::WI;
   static constexpr int LOADS = XI + WI + T::SZI;
   static_assert(XI * WAVES * 8 == BM, "whole x load instructions");
   static_assert(S * STAGE <= 160 * 1024, "LDS");
@@ -126,7 +127,7 @@ struct GemmCfg {
 // partials in memory that a split over workgroups costs.
 //
 // NARROW: N is only a multiple of 4. e4m3 K rows are then 4-byte aligned and come as dword loads to
-// LDS (four times as many), int4 scale and zero rows 8-byte aligned and come as dwords of 32 lanes.
+// LDS (four times as many).
 template <WFmt F, int WAVES, int MT, int S, int KG, bool SW, bool NARROW = false>
 __device__ __forceinline__ void gemm_body(const ldk::GemmArgs& a, int kps, float* partial, int mfast) {
   using C = GemmCfg<F, WAVES, MT, S, NARROW>;
@@ -219,7 +220,7 @@ __device__ __forceinline__ void gemm_body(const ldk::GemmArgs& a, int kps, float
   const int gsh = kInt4 ? __builtin_ctz(a.group_size) - 6 : 0;  // log2(K-steps per group)
   const uint32_t szb = kInt4 ? (uint32_t)(a.K / a.group_size) * (uint32_t)a.N * 2u : 0u;
   const u32x4 sb = raw_rsrc(a.s, szb), zb = raw_rsrc(a.z, szb);
-  const uint32_t szoff = 2u * (uint32_t)(n0 + (NARROW ? 2 * (lane & 31) : 8 * (lane & 7)));
+  const uint32_t szoff = 2u * (uint32_t)(n0 + 8 * (lane & 7));
 
   auto issue = [&](unsigned char* stage, int kstep) {
     const int ks = kbeg + kstep;
@@ -228,19 +229,14 @@ __device__ __forceinline__ void gemm_body(const ldk::GemmArgs& a, int kps, float
       dma_buffer16(xb, xoff[i], (uint32_t)(ks * kXRow), lds_addr(stage + 8 * (C::XI * wave + i) * kXRow));
 #pragma unroll
     for (int i = 0; i < WI; ++i) {
-      if constexpr (NARROW && !kInt4)
+      if constexpr (NARROW)
         dma_buffer4(wb, woff[i], (uint32_t)ks * wstep, lds_addr(stage + C::WOFF + T::WBYTES * wave + 256 * i));
       else
         dma_buffer16(wb, woff[i], (uint32_t)ks * wstep, lds_addr(stage + C::WOFF + T::WBYTES * wave + 1024 * i));
     }
     if constexpr (kInt4) {
       const uint32_t g = 2u * (uint32_t)(ks >> gsh) * (uint32_t)a.N;
-      if constexpr (NARROW) {
-        if (lane < 32) {
-          dma_buffer4(sb, g + szoff, 0u, lds_addr(stage + C::SZOFF + 256 * wave));
-          dma_buffer4(zb, g + szoff, 0u, lds_addr(stage + C::SZOFF + 256 * wave + 128));
-        }
-      } else if (lane < 8) {  // one instruction each; lanes 8-63 idle (every wave has lanes 0-7 active)
+      if (lane < 8) {  // one instruction each; lanes 8-63 idle (every wave has lanes 0-7 active)
         dma_buffer16(sb, g + szoff, 0u, lds_addr(stage + C::SZOFF + 256 * wave));
         dma_buffer16(zb, g + szoff, 0u, lds_addr(stage + C::SZOFF + 256 * wave + 128));
       }
@@ -481,13 +477,7 @@ __global__ __launch_bounds__(WAVES * KG * 64) __attribute__((amdgpu_waves_per_eu
   gemm_body<WFmt::kE4M3, WAVES, MT, S, KG, false>(a, kps, partial, mfast);
 }
 
-// The same GEMMs for N a multiple of 4 only.
-template <int WAVES, int MT, int S, int KG>
-__global__ __launch_bounds__(WAVES * KG * 64) __attribute__((amdgpu_waves_per_eu(2))) void w4a16_gemm_narrow_kernel(
-    ldk::GemmArgs a, int kps, float* partial, int mfast) {
-  gemm_body<WFmt::kInt4, WAVES, MT, S, KG, false, true>(a, kps, partial, mfast);
-}
-
+// The e4m3 GEMM for N a multiple of 4 only.
 template <int WAVES, int MT, int S, int KG>
 __global__ __launch_bounds__(WAVES * KG * 64) __attribute__((amdgpu_waves_per_eu(2))) void w8a16_gemm_narrow_kernel(
     ldk::GemmArgs a, int kps, float* partial, int mfast) {
@@ -652,14 +642,10 @@ int launch(const ldk::GemmArgs& a, int splits, int mfast, hipStream_t s) {
     }
   }
   if (a.swiglu) return ldk::fail(LDK_ERR_UNSUPPORTED, "gemm: SwiGLU epilogue not built for %d x %d tiles", WAVES, MT);
-  const bool narrow = a.N % (F == WFmt::kInt4 ? 8 : 16) != 0;
   if constexpr (F == WFmt::kInt4) {
-    if (narrow)
-      w4a16_gemm_narrow_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
-    else
-      w4a16_gemm_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
+    w4a16_gemm_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
   } else {
-    if (narrow)
+    if (a.N % 16)
       w8a16_gemm_narrow_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
     else
       w8a16_gemm_kernel<WAVES, MT, S, KG><<<grid, WAVES * KG * 64, 0, s>>>(a, kps, partial, mfast);
@@ -700,7 +686,7 @@ namespace ldk {
 bool gemm_supported(WFmt f, int64_t M, int64_t N, int64_t K, int group_size, int64_t ldx, bool narrow) {
   if (M <= 0 || N <= 0 || K <= 0 || K % kStep) return false;
   if (f == WFmt::kInt4) {
-    if (group_size < kStep || (group_size & (group_size - 1)) || K % group_size || N % (narrow ? 4 : 8)) return false;
+    if (group_size < kStep || (group_size & (group_size - 1)) || K % group_size || N % 8) return false;
     // scales and zeros are read through 32-bit buffer offsets
     if ((K / group_size) * N * 2 >= (int64_t(1) << 31)) return false;
   } else if (N % (narrow ? 4 : 16)) {
@@ -754,7 +740,8 @@ const char* gemm_kernel_name(WFmt f, int64_t M, int64_t N, int64_t K, int block_
   // the library's workspace (64 MiB) bounds the split, as in a call through ldk_*_matmul
   const GemmShape sh = pick_shape(f, M, N, K, block_n, 0, int64_t(64) << 20);
   static thread_local char buf[64];
-  snprintf(buf, sizeof(buf), "%s_gemm_kernel<%d, %d, %d, %d>", f == WFmt::kInt4 ? "w4a16" : "w8a16", sh.waves, sh.mt,
+  snprintf(buf, sizeof(buf), "%s_kernel<%d, %d, %d, %d>",
+           f == WFmt::kInt4 ? "w4a16_gemm" : N % 16 ? "w8a16_gemm_narrow" : "w8a16_gemm", sh.waves, sh.mt,
            stages_of(f, sh.waves, sh.mt, sh.kg), sh.kg);
   return buf;
 }

@@ -1822,9 +1822,7 @@ static constexpr int64_t kGemmRows = 64;
 static constexpr int64_t kGemmWideRows = 32;  // from this many rows on shapes of N >= 8192
 
 static bool gemm_applies(int64_t M, int64_t N, int64_t K, int group_size, int64_t ldx, const void* out, int64_t ldo, bool forced) {
-  // the library's own choice takes N % 8 == 4 too from 1e9 multiply-adds (the GEMM's narrow variant;
-  // 4124x3968, blocks against GEMM: M = 658 81 / 48 us, 3055 330 / 108)
-  return (forced || M > 16) && ldk::gemm_supported(ldk::WFmt::kInt4, M, N, K, group_size, ldx, !forced && M * N * K >= 1000000000) && (!out || ldk::aligned(out, 8)) &&
+  return (forced || M > 16) && ldk::gemm_supported(ldk::WFmt::kInt4, M, N, K, group_size, ldx) && (!out || ldk::aligned(out, 8)) &&
          ldo % 4 == 0;
 }
 
@@ -1846,16 +1844,17 @@ static bool uses_gemm(int64_t M, int64_t N, int64_t K, int group_size, int64_t l
   // 64: 12.0 / 22.6 us on the blocks, 10.5 / 15.3 on the GEMM's 32-row tiles; M = 17: 9.5 against
   // 10.3)
   if (M < (N >= 8192 ? kGemmWideRows : kGemmRows + 1)) return false;
-  const bool large = N * K >= 20000000;
   // narrow shapes from 257 rows where the blocks need more than 256 workgroups, and from 512 rows:
   // past 256 workgroups the blocks lose a round (qkv M = 288 / 384 on 9 / 12 x 32 blocks: 14.9 /
   // 15.0 us against 10.3 on the GEMM; down M = 384 / 448: 47.7 / 47.4 against 28.8 / 29.7), below
   // it they keep the lead (down M = 288 on 9 x 24 blocks: 25.8 against 33.0; M = 256: 25.6 against
   // 28.4; qkv M = 256 on 8 x 32: 8.5 against 10.3)
   const int64_t blocks = (N + 63) / 64 * ((M + 31) / 32);
-  // from 20M weights already past 160 rows (4096x14336 M = 200: 70.9 us on the blocks, 53.8 on the
-  // GEMM; 6144x4096 37.8 and 29.3, but M = 140 26.0 and 28.6)
-  if (!(N >= 8192 || M >= 512 || (M > (large ? 160 : 256) && blocks > 256))) return false;
+  // The GEMM rounds each dequantized weight to fp16, the blocks round none (against 64 bits 2.76e-4
+  // and 2.07e-4 at 4100x4096): rows that the blocks have are not handed over for their time alone
+  // (4096x14336 M = 200 would take 53.8 instead of 70.9 us, and N % 8 == 4, 4124x3968 M = 658, 48
+  // instead of 81).
+  if (!(N >= 8192 || M >= 512 || (M > 256 && blocks > 256))) return false;
   return gemm_applies(M, N, K, group_size, ldx, out, ldo, false);
 }
 

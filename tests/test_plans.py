@@ -1,0 +1,15 @@
+"""What the library's own choice runs for a shape (the plan queries need no GPU): the lines that the
+sources draw from measured times, on both sides."""
+
+import pytest
+
+from kernels import fp8, w4a16
+
+
+@pytest.mark.parametrize("M,N,K", [(1030, 1012, 2048), (130, 17924, 1024), (200, 4096, 14336), (161, 6144, 4096),
+                                   (256, 8064, 2560)])
+def test_int4_rows_stay_on_the_row_blocks(M, N, K):
+    """N % 8 == 4, and up to 256 rows on narrow weights: the blocks round no weight, the GEMM rounds
+    each to fp16."""
+    assert w4a16.config_for(M, N, K).startswith("mfma,")
+    assert w4a16.kernel_name(M, N, K).startswith("w4a16_mfma_kernel<")
