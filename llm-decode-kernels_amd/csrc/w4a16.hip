@@ -1394,16 +1394,14 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int gsh_rows, int block_n, int s
   // kernels, which dequantize every weight as dequantize_ref does.
   // Two rows on a narrow shape of more than 2 MB (down) also take the MFMA kernel, split K ten
   // ways: 4.9 against 5.4 us for the two-row VALU kernel (wide shapes keep it: gate_up 5.7 us).
+  // Large weights are no reason for one row, or for two on a wide shape, to leave the VALU kernel:
+  // its error against 64 bits is the smaller (14336x4096 2.07e-4 against 2.08e-4, 28672x4096 M = 2
+  // 2.08e-4 against 2.09e-4: the MFMA kernel's sums of x (1024 + q) cancel), and the MFMA kernel is
+  // faster only where its tiles fill nearly all CUs (M = 1, weights from HBM, 14336x4096 11.5 against
+  // 9.4 us, 4096x14336 12.9 against 9.7) and slower elsewhere (8064x11008 12.0 against 13.2,
+  // 17920x7168 18.4 against 22.5, 151936x1536 26.4 against 36.0).
   const bool narrow_long = N < 128 * 128 && wbytes > (2 << 20);
-  // One and two rows take the MFMA kernel from 48M weights: the VALU kernels' tiles of 32 columns
-  // over a long K then run in several rounds of workgroups (M = 1 / 2: 28672x4096 17.0 / 18.3 ->
-  // 15.4 / 15.4 us, 14336x4096 11.0 / 11.6 -> 8.6 / 8.6, 4096x14336 M = 1 12.4 -> 9.1; 6144x4096, 25M
-  // weights, 5.6 against 6.1), unless its 64-column tiles leave a quarter of the CUs idle (10240x8192,
-  // 160 tiles, M = 1 12.4 against 13.5).
-  const int64_t t64 = (N + 63) / 64;
-  const bool few_large = M <= 2 && N * K >= 48000000 && block_n == 0 && split_k <= 0 && !(flags & LDK_FACTORED) &&
-                         (M == 2 || t64 > 256 || t64 * (256 / t64) >= 192);
-  const bool mfma_auto = M > 8 || (!(flags & LDK_EXACT) && (M > 2 || (M == 2 && narrow_long && block_n == 0) || few_large) &&
+  const bool mfma_auto = M > 8 || (!(flags & LDK_EXACT) && (M > 2 || (M == 2 && narrow_long && block_n == 0)) &&
                                    (block_n == 0 || block_n >= 64));
   const bool mfma = (flags & LDK_PATH_MFMA) || (mfma_auto && !(flags & LDK_PATH_VALU));
   const bool m1 = !mfma && !(flags & LDK_EXACT) && M <= 2;  // the factored VALU kernel
@@ -1441,6 +1439,7 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int gsh_rows, int block_n, int s
   // rows) 8.8 / 15.1 -> 8.8 / 10.6, 4096x14336 in 4 9.2 / 23.1 -> 9.1 / 11.2, 2560x11648 in 6 M = 16
   // 9.5 -> 8.3, 8192x8192 in 2 12.5 / 13.5 -> 9.8 / 11.6; from 13 rows not where a short K would be
   // split (8064x2560 in 2 7.2 against 6.5).
+  const int64_t t64 = (N + 63) / 64;
   const bool large = mfma && M <= 16 && block_n == 0 && split_k <= 0 && N * K >= 20000000 && t64 <= 256 &&
                      (M <= 12 || K >= 4096 || t64 > 128);
   if (mfma) {  // 128 columns on shapes wide enough to fill the CUs with them, else 64 (and 64 for
@@ -2169,7 +2168,7 @@ extern "C" int ldk_w4a16_rmsnorm_matmul(const void* x, const void* residual, voi
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_rmsnorm_matmul: norm_weight, residual and residual_out must be 16-byte aligned");
   if (workspace_bytes && (!workspace || !ldk::aligned(workspace, 256)))
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_rmsnorm_matmul: workspace must be a 256-byte aligned pointer");
-  Plan p = make_plan(1, N, K, gsh_rows, 0, 0, LDK_PATH_VALU, workspace ? (size_t)workspace_bytes : 0);
+  Plan p = make_plan(1, N, K, gsh_rows, 0, 0, 0, workspace ? (size_t)workspace_bytes : 0);
   if (p.full) {  // whole tiles: every workgroup then reads the whole row, which its statistic needs
     p.full = 0;
     p.splits = 1;
@@ -2189,7 +2188,7 @@ extern "C" int ldk_w4a16_swiglu_matmul(const void* gate_up, const int32_t* qweig
   if (st) return st;
   if (workspace_bytes && (!workspace || !ldk::aligned(workspace, 256)))
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_swiglu_matmul: workspace must be a 256-byte aligned pointer");
-  const Plan p = make_plan(1, N, K, gsh_rows, 0, 0, LDK_PATH_VALU, workspace ? (size_t)workspace_bytes : 0);
+  const Plan p = make_plan(1, N, K, gsh_rows, 0, 0, 0, workspace ? (size_t)workspace_bytes : 0);
   const W4Args a{(const half_t*)gate_up, 2 * K, (const uint32_t*)qweight, (const half_t*)scales, (const half_t*)zeros,
                  (const half_t*)bias, (half_t*)out, N, 1, (int)N, (int)K, gsh_rows};
   return launch_plan(a, p, workspace, (hipStream_t)stream, kProSwiglu, ProArgs{});
@@ -2205,7 +2204,7 @@ extern "C" int ldk_w4a16_swiglu_matmul(const void* gate_up, const int32_t* qweig
 
 namespace {
 Plan residual_stats_plan(int64_t N, int64_t K, int gsh_rows, size_t ws) {
-  Plan p = make_plan(1, N, K, gsh_rows, 0, 0, LDK_PATH_VALU, ws);
+  Plan p = make_plan(1, N, K, gsh_rows, 0, 0, 0, ws);
   p.full = 0;
   p.splits = 1;
   p.gps = (int)((K / 8) >> gsh_rows);
@@ -2302,7 +2301,7 @@ extern "C" int ldk_w4a16_rmsnorm_stats_matmul(const void* h, const float* row_st
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_rmsnorm_stats_matmul: norm_weight 16-byte, row_stats 4-byte aligned");
   if (workspace_bytes && (!workspace || !ldk::aligned(workspace, 256)))
     return ldk::fail(LDK_ERR_ALIGN, "w4a16_rmsnorm_stats_matmul: workspace must be a 256-byte aligned pointer");
-  const Plan p = make_plan(1, N, K, gsh_rows, 0, 0, LDK_PATH_VALU, workspace ? (size_t)workspace_bytes : 0);
+  const Plan p = make_plan(1, N, K, gsh_rows, 0, 0, 0, workspace ? (size_t)workspace_bytes : 0);
   const W4Args a{(const half_t*)h, K, (const uint32_t*)qweight, (const half_t*)scales, (const half_t*)zeros,
                  (const half_t*)bias, (half_t*)out, N, 1, (int)N, (int)K, gsh_rows};
   const ProArgs pa{nullptr, nullptr, (const half_t*)norm_weight, eps, const_cast<float*>(row_stats), nstats};

@@ -10,8 +10,8 @@ libldk_amd.so whose tile and K-split come from the library's per-shape table:
   per-device workspace, all within the one launch, so there is no zero-fill or cast launch (the
   reference's split paths add two elementwise launches, w4a16.py:218-219,272-275);
 - M = 1 and M = 2 use the FACTORED inner loop s * (sum x*q - z * sum x) (w4a16.py:116-119) on
-  the VALU, each packed word decoded once for both rows; from 3 rows (and from 48M weights for one
-  and two rows) the MFMA kernel computes the same factored form on the matrix cores. `config={"FACTORED": False}` (EXACT, M <= 8) instead
+  the VALU, each packed word decoded once for both rows; from 3 rows the MFMA kernel computes the
+  same factored form on the matrix cores. `config={"FACTORED": False}` (EXACT, M <= 8) instead
   dequantizes each weight exactly as dequantize_ref and accumulates with v_dot2_f32_f16.
 
 Prefill shapes (the reference's Triton tensor-core GEMM path, w4a16.py:264-268) run hand-written

@@ -13,3 +13,10 @@ def test_int4_rows_stay_on_the_row_blocks(M, N, K):
     each to fp16."""
     assert w4a16.config_for(M, N, K).startswith("mfma,")
     assert w4a16.kernel_name(M, N, K).startswith("w4a16_mfma_kernel<")
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 14336, 4096), (1, 8064, 11008), (1, 151936, 1536), (2, 40960, 2560), (2, 28672, 4096)])
+def test_int4_one_and_two_rows_stay_on_the_valu_kernel(M, N, K):
+    """However large the weights: its error is the smaller, and the quantized lm_head and most other
+    shapes are slower on the MFMA kernel."""
+    assert w4a16.config_for(M, N, K).startswith("valu,")
