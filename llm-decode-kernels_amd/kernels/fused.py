@@ -9,8 +9,8 @@ launch. The staged activations follow the standalone kernels' rounding steps (`k
 `kernels.swiglu`); SwiGLU's are bit-identical to them, RMSNorm's can differ from them by one fp16
 ulp, because the row's sum of squares is reduced in another order.
 
-Rows other than one (prefill), group sizes other than 128 and projections past FUSED_NORM_MAX_N or
-FUSED_MAX_WEIGHTS run the two ops back to back.
+Rows other than one (prefill), group sizes other than 128 and projections that norm_fuses leaves out
+run the two ops back to back.
 """
 
 from __future__ import annotations
@@ -23,16 +23,21 @@ from kernels.swiglu import swiglu_fused
 from kernels.w4a16 import w4a16_matmul
 
 FUSED_GROUP_SIZE = 128
-# Widest projection that rmsnorm_w4a16_matmul fuses. Every workgroup of the fused launch forms
-# the row statistic itself (its own loads and a barrier) and the launch takes whole column tiles,
-# which costs little on one round of tiles and grows with the rounds. Graph-timed, fused against
-# the norm as a launch of its own: 2048x1536 3.6 / 5.5 us, 17920x1536 7.4 / 7.5, 18688x2176
-# 10.9 / 10.0, 28672x4096 24.2 / 17.8, the 151936-row quantized lm_head 33.4 / 26.5.
-FUSED_NORM_MAX_N = 18432
-# Weights (N * K) from which one row's projection runs the library's matrix-core plan, which takes
-# no prologue: the norm or activation is then a launch of its own (swiglu into 4096x14336 12.7 us
-# fused, 11.0 in two launches; 2560x11648, 30M weights, 6.4 against 8.1).
-FUSED_MAX_WEIGHTS = 48_000_000
+# Widest projection that rmsnorm_w4a16_matmul fuses, at up to 1024 inputs (norm_fuses).
+FUSED_NORM_MAX_N = 65536
+
+
+def norm_fuses(N: int, K: int) -> bool:
+    """Whether one row's norm rides in the projection's launch. Every workgroup of the fused launch
+    forms the row statistic itself (its own loads and a barrier, both longer with K) and the launch
+    takes whole column tiles, which costs little on the first round of workgroups (256 tiles of 32
+    columns) and grows with the rounds; a launch of its own costs about 2.3 us. Fused against two
+    launches, us, weights from HBM: 8192 x 1536 / 4096 / 8192 4.8 / 5.9, 8.3 / 8.6, 11.8 / 13.1;
+    32768 and 65536 x 1024 7.1 / 8.1, 10.7 / 11.8; 24576 x 1536 / 2048 8.6 / 8.8, 10.0 / 10.4; 32768 x
+    1536 10.4 / 10.2; 17920 x 2560 11.6 / 10.7; 12288 and 28672 x 4096 13.7 / 11.4, 25.4 / 20.8; the
+    quantized lm_head 151936 x 1536 36.7 / 28.6."""
+    eighths = 8 if K <= 1024 else 3 if K <= 2048 else 1  # of FUSED_NORM_MAX_N: 65536, 24576, 8192
+    return 8 * N <= eighths * FUSED_NORM_MAX_N
 
 
 def _aligned(*ts) -> bool:
@@ -49,8 +54,7 @@ def rmsnorm_w4a16_matmul(x, weight, eps, residual, qweight, scales, zeros, group
     N = qweight.shape[1]
     rows = x.numel() // K
     fuse = (rows == 1 and group_size == FUSED_GROUP_SIZE and x.dtype == torch.float16
-            and weight.dtype == torch.float16 and x.is_cuda and N <= FUSED_NORM_MAX_N
-            and N * K < FUSED_MAX_WEIGHTS
+            and weight.dtype == torch.float16 and x.is_cuda and norm_fuses(N, K)
             and _aligned(x, weight, residual, qweight))
     if not fuse:
         if residual is None:
@@ -86,8 +90,7 @@ def swiglu_w4a16_matmul(gate_up, qweight, scales, zeros, group_size=128, bias=No
     N = qweight.shape[1]
     rows = gate_up.numel() // K2
     fuse = (rows == 1 and group_size == FUSED_GROUP_SIZE and gate_up.dtype == torch.float16
-            and gate_up.is_cuda and _aligned(gate_up, qweight) and K % 8 == 0
-            and N * K < FUSED_MAX_WEIGHTS)
+            and gate_up.is_cuda and _aligned(gate_up, qweight) and K % 8 == 0)
     if not fuse:
         return w4a16_matmul(swiglu_fused(gate_up), qweight, scales, zeros, group_size, bias)
     assert K2 % 2 == 0 and qweight.shape[0] * 8 == K
@@ -115,8 +118,10 @@ def linear_rmsnorm_w4a16_matmul(x, qweight1, scales1, zeros1, bias1, residual, w
     y2 = linear2(rmsnorm(h) * weight). One row runs two launches
     (ldk_w4a16_matmul_residual_stats, ldk_w4a16_rmsnorm_stats_matmul): the residual add and the
     row's per-tile sums of squares come out of the first projection's epilogue, so the second
-    one forms the norm in its x staging without reducing the row itself. Other rows run
-    w4a16_matmul then rmsnorm_w4a16_matmul."""
+    one forms the norm in its x staging without reducing the row itself, which pays at every width
+    (o and gate_up in us, weights from HBM, against three launches: hidden 1536 to 17920 columns
+    11.1 / 12.4, 4096 to 28672 24.6 / 25.7, 8192 to 28672 41.6 / 43.1). Other rows run w4a16_matmul
+    then rmsnorm_w4a16_matmul."""
     K1 = x.shape[-1]
     N1 = qweight1.shape[1]
     rows = x.numel() // K1

@@ -50,6 +50,12 @@ def test_rmsnorm_matmul(N, K, bias, with_res, monkeypatch):
     import kernels.fused as fused_mod
 
     monkeypatch.setattr(fused_mod, "FUSED_NORM_MAX_N", 1 << 30)  # the fused launch at every N
+
+    def composed(*_, **__):
+        raise AssertionError("the two-launch composition ran")
+
+    monkeypatch.setattr(fused_mod, "rmsnorm", composed)
+    monkeypatch.setattr(fused_mod, "w4a16_matmul", composed)
     qw, s, z, b = _weights(N, K, 11, bias)
     x, r, w = cases.rmsnorm_case(1, K, 12)
     res = r.cuda() if with_res else None
@@ -89,8 +95,14 @@ def test_rmsnorm_matmul_wide_runs_two_launches():
     assert torch.equal(h, res2) and torch.equal(y, w4a16_matmul(h2, qw, s, z, 128))
 
 
-@pytest.mark.parametrize("N,K", [(1536, 8960), (1536, 1536), (256, 8960), (4096, 2048)])
-def test_swiglu_matmul(N, K):
+@pytest.mark.parametrize("N,K", [(1536, 8960), (1536, 1536), (256, 8960), (4096, 2048), (4096, 14336)])
+def test_swiglu_matmul(N, K, monkeypatch):
+    import kernels.fused as fused_mod
+
+    def composed(*_, **__):
+        raise AssertionError("the two-launch composition ran")
+
+    monkeypatch.setattr(fused_mod, "w4a16_matmul", composed)
     qw, s, z, b = _weights(N, K, 21, bias=(N == 256))
     gu = cases.swiglu_case(1, K, 22)
     y = swiglu_w4a16_matmul(gu.cuda(), qw, s, z, 128, None if b is None else b.cuda())

@@ -3,7 +3,7 @@ sources draw from measured times, on both sides."""
 
 import pytest
 
-from kernels import fp8, w4a16
+from kernels import fp8, fused, w4a16
 
 
 @pytest.mark.parametrize("M,N,K", [(1030, 1012, 2048), (130, 17924, 1024), (200, 4096, 14336), (161, 6144, 4096),
@@ -20,3 +20,10 @@ def test_int4_one_and_two_rows_stay_on_the_valu_kernel(M, N, K):
     """However large the weights: its error is the smaller, and the quantized lm_head and most other
     shapes are slower on the MFMA kernel."""
     assert w4a16.config_for(M, N, K).startswith("valu,")
+
+
+@pytest.mark.parametrize("N,K,fuses", [(8192, 8192, True), (24576, 1024, True), (65536, 512, True), (20480, 1536, True),
+                                       (24576, 2048, True), (28672, 1536, False), (12288, 4096, False),
+                                       (17920, 2560, False), (151936, 1024, False), (151936, 1536, False)])
+def test_one_row_norm_in_the_projections_launch(N, K, fuses):
+    assert fused.norm_fuses(N, K) == fuses
