@@ -1047,8 +1047,6 @@ static bool w8_uses_gemm(int64_t M, int64_t N, int64_t K, int64_t ldx, const voi
   // wide shapes (N >= 8192) from 17 rows: the 16-row blocks re-read all of their e4m3 weights per
   // block (gate_up M = 17 / 32 / 64: 16.9 / 20.3 / 29.7 us on the blocks, 10.9 / 11.2 / 15.5 on the
   // GEMM's 32-row tiles)
-  // (from 20M weights past 32 rows on narrow shapes too: M = 33 4096x14336 41 -> 29 us, 6144x4096
-  // 24 -> 16)
   const bool large = N * K >= 20000000;
   if (M <= (N >= 8192 ? 16 : large ? 32 : kW8GemmRows) || block_n || split_k || (flags & (LDK_PATH_VALU | LDK_PATH_MFMA))) return false;
   // narrow shapes past 64 rows keep the blocks while they fit in 256 workgroups: short K on
@@ -1056,9 +1054,17 @@ static bool w8_uses_gemm(int64_t M, int64_t N, int64_t K, int64_t ldx, const voi
   // against 9.7; qkv M = 160, 320 workgroups, 13.4 against 10.2), long K while they still split K
   // at least twice (down M = 96 / 128 / 160: 19.8 / 23.4 / 23.6 against 26.0 / 26.5 / 24.2; M = 192
   // in whole K 41.0 against 24.6)
-  if (N < 8192 && !large) {
-    const int64_t blocks = (M + 15) / 16;
-    if (w8_short_k(K) ? (N + 63) / 64 * blocks <= 256 : (N + 127) / 128 * blocks <= 128) return false;
+  // From 20M weights, where K is long, already past 32 rows, and the blocks keep the shapes on which they
+  // split K so often that they still stream from most CUs. Weights from HBM, tiles of 128 columns times
+  // 16-row blocks, blocks against GEMM: 36 (1536x14336 M = 33) 18.6 / 33.1, 48 (2048x13312 M = 33) 19.4 /
+  // 31.4, 72 (3072x8192 M = 48) 20.8 / 25.4, 80 (2560x13312 M = 64) 30.6 / 32.5; 96 (4096x14336 M = 33)
+  // 35 / 29, (1536x13312 M = 128) 34.4 / 35.9, (2048x13312 M = 96) 35 / 29; 144 (6144x4096 M = 33) 24 / 17.
+  // Rows of 8- and 4-byte alignment slow the blocks down more than the GEMM: N = 1544 at 39 / 65
+  // 0.82 / 1.09 of the GEMM's time, 2056 at 51 / 68 0.95 / 1.29; 1028 at 27 / 36 0.65 / 0.97, 1540 at 39 0.99.
+  if (N < 8192) {
+    const int64_t blocks = (M + 15) / 16, wide = (N + 127) / 128 * blocks;
+    const int64_t first = N % 8 ? 36 : N % 16 ? 60 : N < 2048 ? 104 : 96;  // of the GEMM's
+    if (large ? wide < first : w8_short_k(K) ? (N + 63) / 64 * blocks <= 256 : wide <= 128) return false;
   }
   // N % 16 != 0 (the GEMM's narrow variant, dword loads) from 1e9 multiply-adds: 4120x3968, blocks
   // against GEMM, M = 200 65 / 27 us, 3055 838 / 105; 17924x1536 M = 3055 2298 / 174

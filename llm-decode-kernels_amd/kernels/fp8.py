@@ -9,9 +9,10 @@ GPU, results returned on the CPU). Decode shapes run the wave64 VALU GEMV with a
 split-K at M = 1 and the MFMA kernel (in-register byte transpose, exact e4m3 -> fp16) from 2 rows.
 Prefill rows (the reference's tensor-core GEMM, fp8.py:42-91 run at fp8.py:221-222) run
 hand-written kernels at every row count: the MFMA kernel in 16-row blocks (17-64 rows, and on
-narrow shapes under 20 MB of weights while the blocks fit in 256 workgroups: short K on 64-column tiles with K split
-toward 256 workgroups, long K while they still split K at least twice), else (and from 17 rows on
-wide shapes, N >= 8192) the prefill GEMM (csrc/prefill.hip: 32/64/128-row tiles, e4m3 tiles
+narrow shapes while the blocks fit in 256 workgroups: short K on 64-column tiles with K split
+toward 256 workgroups, long K while they still split K at least twice; from 20M weights, past 32 rows,
+under 96 tiles of 128 columns x 16 rows), else (and from 17 rows on wide shapes, N >= 8192) the
+prefill GEMM (csrc/prefill.hip: 32/64/128-row tiles, e4m3 tiles
 transposed and converted to fp16 in registers, column scale after the K loop, K split over
 workgroups for long K).
 `config={"prefill": "gemm" | "blocks"}` forces one of them; "native" is the library's choice.

@@ -27,3 +27,13 @@ def test_int4_one_and_two_rows_stay_on_the_valu_kernel(M, N, K):
                                        (17920, 2560, False), (151936, 1024, False), (151936, 1536, False)])
 def test_one_row_norm_in_the_projections_launch(N, K, fuses):
     assert fused.norm_fuses(N, K) == fuses
+
+
+@pytest.mark.parametrize("M,N,K,path", [(33, 2048, 13312, "mfma"), (48, 3072, 8192, "mfma"), (64, 2560, 13312, "mfma"),
+                                        (65, 1536, 14336, "mfma"), (128, 1536, 13312, "mfma"), (140, 1536, 13312, "gemm"),
+                                        (33, 4096, 14336, "gemm"), (96, 2048, 12288, "gemm"), (33, 6144, 4096, "gemm"),
+                                        (48, 1028, 20480, "mfma"), (65, 1028, 20480, "gemm"), (64, 1544, 14336, "mfma"),
+                                        (65, 1544, 14336, "gemm"), (48, 2052, 10240, "gemm")])
+def test_e4m3_hand_over_to_the_gemm_on_large_narrow_weights(M, N, K, path):
+    """At 96 tiles of 128 columns x 16 rows; rows of less alignment at 60 and 36."""
+    assert fp8.config_for(M, N, K).startswith(path + ",")
