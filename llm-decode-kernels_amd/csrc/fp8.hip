@@ -768,13 +768,22 @@ W8Plan make_w8_mfma_plan(int64_t M, int64_t N, int64_t K, int block_n, int split
   // plans below, 28672x4096 in 1 split (8 / 3 before) 27.5 / 38.9 -> 24.7 / 27.6 us, 4096x14336 in 8
   // (10 of 64 columns) 20.8 / 28.4 -> 13.8 / 18.2, 11264x2048 in 2 (4 / 2 of 64) 9.7 / 12.9 -> 8.1 /
   // 11.2; under 14 MB the plans below win (1536x8960 in 10 of 64 6.2 / 7.2 against 7.4 / 9.9). From 5
-  // rows at most 8 splits (3072x7680 in 10: M = 13 12.1 against 11.7 us in 5 of 64 columns); up to 4
-  // rows not where whole tiles would leave a quarter of the CUs idle and the pieces of 16 steps
-  // below do not (20480x2560, 160 tiles: 16.9 against 15.0).
+  // rows at most 8 splits (3072x7680 in 10: M = 13 12.1 against 11.7 us in 5 of 64 columns). Not where
+  // the plans below fill the CUs in one round (times of theirs over this plan's, weights from HBM):
+  //  - 64-column tiles in splits of one pass number at most 256: then pieces of about 24 steps lose
+  //    their returning atomics (7936x2560 M = 4 / 13 0.87 / 0.82, 4096x5632 M = 13 0.94, 5376x4096 M = 5 0.85;
+  //    just past 256, 6144x3584 and 4096x7680, 1.45 and 1.6), but for 2 and 3 rows on 24 tiles and more,
+  //    which have few outputs to add (5120x4096 1.19 / 1.14, 4096x6144 1.13 / 1.06, 7936x2560 M = 2 0.97);
+  //  - whole tiles would leave CUs idle. Up to 4 rows under 192 workgroups, where the pieces of 16 steps
+  //    do not (20480x2560, 160 tiles: 16.9 against 15.0 us). From 5 rows under 176, where K is more than
+  //    3072, past 12 rows 5120 (17920 / 20480x7168 M = 5 0.88 / 0.98, 17408x4096 M = 8 / 13 0.90 / 0.97,
+  //    17920x3072 and 5120 M = 13 1.24 and 1.14; 22528, 176 tiles, 1.05-1.3 at any K).
   const int64_t wide_tiles = (N + 127) / 128, wide_splits = std::max<int64_t>(1, std::min<int64_t>(256 / wide_tiles, steps / 8));
+  const bool one_round = (N + 63) / 64 * ((steps + 6 * p.nw - 1) / (6 * p.nw)) <= 256 && !(M <= 3 && wide_tiles >= 24);
+  const bool idle = wide_tiles >= 128 && wide_tiles * wide_splits < (M <= 4 ? 192 : 176) &&
+                    (M <= 4 || steps > (M <= 12 ? 96 : 160));
   const bool stream = M <= 16 && block_n == 0 && split_k <= 0 && N % 8 == 0 && steps > 48 && wide_tiles <= 256 &&
-                      N * K >= 20000000 &&
-                      (M <= 4 ? wide_tiles < 128 || wide_tiles * wide_splits >= 192 : wide_splits <= 8);
+                      N * K >= 20000000 && !one_round && !idle && (M <= 4 || wide_splits <= 8);
   if (stream) p.ln = 8;
   const int64_t tiles = (N + 16 * p.ln - 1) / (16 * p.ln);
   const int64_t one_pass = (steps + 6 * p.nw - 1) / (6 * p.nw);  // fewest splits of one pass each

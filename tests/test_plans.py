@@ -37,3 +37,17 @@ def test_one_row_norm_in_the_projections_launch(N, K, fuses):
 def test_e4m3_hand_over_to_the_gemm_on_large_narrow_weights(M, N, K, path):
     """At 96 tiles of 128 columns x 16 rows; rows of less alignment at 60 and 36."""
     assert fp8.config_for(M, N, K).startswith(path + ",")
+
+
+@pytest.mark.parametrize("M,N,K,plan", [(4, 7936, 2560, "block_n=64"), (13, 4096, 5632, "block_n=64"),
+                                        (5, 5376, 4096, "block_n=64"), (2, 1536, 14336, "block_n=64"),
+                                        (2, 5120, 4096, "block_n=128,split_k=6"), (4, 5120, 4096, "block_n=64"),
+                                        (13, 4096, 7680, "block_n=128,split_k=8"), (13, 6144, 3584, "block_n=128,split_k=5"),
+                                        (5, 17920, 7168, "block_n=128,split_k=5"), (12, 18688, 4096, "block_n=128,split_k=3"),
+                                        (13, 17920, 4096, "block_n=128,split_k=1"), (5, 17920, 3072, "block_n=128,split_k=1"),
+                                        (8, 22528, 7168, "block_n=128,split_k=1"), (13, 28672, 4096, "block_n=128,split_k=1"),
+                                        (13, 4096, 14336, "block_n=128,split_k=8")])
+def test_e4m3_decode_rows_on_large_weights(M, N, K, plan):
+    """128-column tiles on at most one workgroup per CU, where the 64-column or split tiles do not
+    fill the CUs in one round themselves."""
+    assert fp8.config_for(M, N, K).startswith("mfma," + plan)
