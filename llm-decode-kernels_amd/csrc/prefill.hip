@@ -577,7 +577,11 @@ GemmShape pick_shape(WFmt f, int64_t M, int64_t N, int64_t K, int block_n, int s
       const int64_t a = ((t * sp + 255) / 256) * best, b = ((t * best + 255) / 256) * sp;
       // equal shares of a K of 192 steps or more: the larger count, up to two workgroups per CU,
       // which hide each other's waits (4096x14336 M = 777: 4 splits instead of 2, e4m3 122 -> 110 us,
-      // int4 135 -> 112; M = 1500: 2 instead of 1, 217 -> 190 and 244 -> 204; 1536x8960, 140 steps, M = 1500 61 against 63)
+      // int4 135 -> 112; M = 1500: 2 instead of 1, 217 -> 190 and 244 -> 204; 1536x8960, 140 steps, M = 1500
+      // 61 against 63). Over 400 shapes of K 12288-20480 the old time is 0.97-1.28 of the new in int4, in
+      // e4m3 0.98-1.26 but for 6 splits on full row tiles (0.94-1.07, level on average) and for 171-191
+      // tiles of 128 x 256, which then stay whole instead of going to 64 x 256 (1.05-1.17, but 0.88-0.97
+      // at N = 5632, 6656 and 11264).
       if (a < b || (a == b && steps >= 192 && t * sp <= 512)) best = sp;
     }
     return (int)best;
