@@ -476,9 +476,13 @@ class QwenRunner:
         self.merge_attention = True  # see forward: the o projection merges the attention's ranges
         # Longest cache whose ranges the o projection merges: it takes at most four, so a range is a
         # quarter of the cache, while decode_attention cuts it into up to 128 and merges them in a
-        # launch of its own. 4-layer decode steps (12/2 heads, W4A16), merged against split: cache
-        # 1024 at pos 371 175 / 182 us, 2048 at 1000 182 / 181, 4096 at 4000 196 / 181, 8192 at 6000
-        # 223 / 186, 32768 at 30000 387 / 208.
+        # launch of its own, which a short context in a long cache pays too (a captured graph has the
+        # same launches at every position). 4-layer decode steps (12/2 heads, W4A16), merged / split, us:
+        # cache 2080 at position 63 / 371 / 1000 / 2000 173 / 177, 181 / 184, 184 / 184, 185 / 185; 8192
+        # at 63 / 200 / 371 / 1000 / 2000 / 8000 173 / 177, 177 / 185, 181 / 186, 199 / 186, 226 / 186,
+        # 226 / 190; 32768 at 63 / 1000 / 30000 174 / 180, 199 / 190, 390 / 211: the first 500 positions of
+        # a long cache are 1-4% slower than merged, the rest up to 85% faster. A program that keeps to short
+        # contexts of a long cache may raise it before it captures.
         self.merge_max_len = 2048
         self.fuse_prompt_act = True  # see forward: SwiGLU in the prompt's gate_up GEMM
         self.warm_weights = True  # see warm_set: the attention launch warms the next weights

@@ -221,6 +221,37 @@ def test_attention_merged_in_o_projection_matches_merge_launch(backend):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("backend", ["ours", "ours_fp8"])
+@pytest.mark.parametrize("max_len", [2048, 2080])
+def test_decode_on_either_side_of_the_merged_caches(backend, max_len):
+    """The decode step of the longest cache whose ranges the o projection merges and of the next one,
+    whose ranges decode_attention merges itself (captured, as a decode loop runs it, replayed at
+    positions with one range live, several and all), against the torch attention on the same cache."""
+    model = _qwen_heads_model("cuda")
+    run = QwenRunner(model, make_backend(backend), max_len=max_len)
+    ref = QwenRunner(model, make_backend(backend), max_len=max_len, attention="torch")
+    assert (run.max_len <= run.merge_max_len) == (max_len == 2048)
+    run.k_cache.normal_(std=0.8)
+    run.vt_cache.normal_(std=0.8)
+    ref.k_cache.copy_(run.k_cache)
+    ref.vt_cache.copy_(run.vt_cache)
+    token, pos = torch.tensor([[7]], device="cuda"), torch.tensor([5], device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run.forward(token, pos)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run.forward(token, pos)
+    for p in (5, 127, 128, 700, max_len - 1, 300):
+        pos.fill_(p)
+        graph.replay()
+        want = ref.forward(token, pos)
+        torch.testing.assert_close(out.float(), want.float(), atol=3e-2, rtol=3e-2)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("backend,T", [("ours", 128), ("ours_fp8", 256)])
 def test_prompt_swiglu_in_gate_up_changes_no_logit(backend, T):
     """The prompt forward on `ours` and `ours_fp8` runs gate_up with SwiGLU in the prefill GEMM's
