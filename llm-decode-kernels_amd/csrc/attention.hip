@@ -799,10 +799,13 @@ __global__ __launch_bounds__(kPWaves * 64) void prefill_attention_kernel(const h
 //
 // What bounds it: about 4 vector instructions per MFMA (exponent, sum, conversion, maximum), which
 // take the wave's issue slots next to the MFMAs' (one MFMA with four fma's between takes 24 cycles
-// on this chip, 16 without), and 32 KB of loads to LDS per 32 positions of a workgroup. Measured
-// (both launches, graph replays, us): 12/2 heads at 3000 tokens 148 -> 71, at 6000 463 -> 172, 1024
-// after 3000 cached 104 -> 61; 28/4 heads at 1500 105 -> 49; 16/16 at 816 44 -> 29 (of these the
-// first launch 10.7 -> 7.6 and 16.3 -> 8.0).
+// on this chip, 16 without), next to 16 KB of loads to LDS per 32 positions of a workgroup. Measured
+// (both launches, graph replays, us; runs on different boxes): 12/2 heads at 3000 tokens 147-157 ->
+// 67-78, at 6000 463-465 -> 172-180, 1024 after 3000 cached 105 -> 61; 28/4 heads at 1500 106 -> 51;
+// 16/16 at 816 44 -> 29 (of these the first launch 10.7 -> 7.6 and 16.3 -> 8.0). Error against 64 bits,
+// four seeds: blocks of 64 level with the 16-token kernel (4.27e-4 at 1024 after 3000), blocks of 128
+// 4.23e-4 against 4.21e-4 at 3000 tokens: their two K groups leave two maxima's numerators exact, not
+// four.
 constexpr int kStepBytes = 2 * kChunk * kHD * 2;  // K and V of one step
 
 template <int CG, int KG, int S>
@@ -1225,7 +1228,8 @@ int attention_partials(const char* what, void* stream, const int64_t* pos, int64
 
 }  // namespace ldk
 
-// Prompt attention (launches prefill_rope_kv_kernel, then prefill_attention_kernel).
+// Prompt attention: prefill_rope_kv_kernel, then prefill_attention_kernel or one of the
+// prefill_attention_block_kernel forms.
 extern "C" int ldk_prefill_attention(const void* qkv, int64_t ldqkv, const int64_t* pos, int64_t T, const float* inv_freq,
                                      void* k_cache, void* vt_cache, void* q_scratch, void* out, int64_t ldo, int nq,
                                      int nkv, int head_dim, int64_t max_len, float scale, void* stream) {
@@ -1267,18 +1271,21 @@ extern "C" int ldk_prefill_attention(const void* qkv, int64_t ldqkv, const int64
   // from 256 workgroups; 64 tokens in four K groups, which halve the longest workgroup's steps but
   // load K and V twice as often, below (28/4 heads at 1500 tokens, 336 workgroups of 128: 51
   // against 64 us; 16/16 at 816, 112: 39 against 36; 12/2 at 1024 after 3000, 96: 73 against 58).
-  // Under 128 workgroups of 64 the 16-token kernel's shorter start wins (12/2 at 511, 96
-  // workgroups: 20.2 against 21.9; at 128: 11.0 against 16.9 us). The block kernels divide by the
-  // scale (positive, not tiny) and store 8 bytes at a time.
+  // Under 160 workgroups of 64 the 16-token kernel's shorter start wins for a prompt from position 0
+  // (times of blocks of 64 over its: 64/8 heads at 128 tokens, 128 workgroups, 1.42, 32/8 at 224 1.32, 28/4
+  // at 320, 140, 1.12, 12/2 at 768, 144, 1.05, 32/8 at 320, 160, 0.99, 12/2 at 896, 168, 0.92; after 1000
+  // cached positions, which the host does not know of, 0.93-1.01 at 128 and 0.77 at 140). The block
+  // kernels take the maximum over unscaled scores, so the scale has to be positive and its product with
+  // a score (below 2^40) finite and no denormal; they store 8 bytes at a time.
   auto launch_blocks = [&](auto kernel, int tokens) {
     const dim3 grid((unsigned)nq, (unsigned)((T + tokens - 1) / tokens));
     kernel<<<grid, 512, 0, s>>>((const half_t*)q_scratch, pos, (int)T, (const half_t*)k_cache, (const half_t*)vt_cache,
                                 (half_t*)out, ldo, nq, nkv, (int)max_len, scale);
     return ldk::check_launch("prefill_attention");
   };
-  if (scale > 1e-20f && ldo % 4 == 0 && ldk::aligned(out, 8) && (T + 63) / 64 <= 65535) {
+  if (scale > 1e-20f && scale < 1e20f && ldo % 4 == 0 && ldk::aligned(out, 8) && (T + 63) / 64 <= 65535) {
     if (nq * ((T + 127) / 128) >= 256) return launch_blocks(prefill_attention_block_kernel<4, 2, 4>, 128);
-    if (nq * ((T + 63) / 64) >= 128) return launch_blocks(prefill_attention_block_kernel<2, 4, 2>, 64);
+    if (nq * ((T + 63) / 64) >= 160) return launch_blocks(prefill_attention_block_kernel<2, 4, 2>, 64);
   }
   const dim3 grid((unsigned)((T + kTile - 1) / kTile), (unsigned)nq);
   prefill_attention_kernel<<<grid, kPWaves * 64, 0, s>>>((const half_t*)q_scratch, pos, (int)T, (const half_t*)k_cache,
