@@ -66,16 +66,13 @@ __device__ __forceinline__ uint16_t from_f32<uint16_t>(float v) {
 // 1293 us on 14336 x 4096 fp16; this 54 us a call, of which the first launch is about 20.
 __device__ __forceinline__ float fp8_scale(float amax) { return fmaxf(amax / 448.0f, 1e-12f); }
 
-// V elements of T per load (1: any base and K). A launch holds fewer than 2^32 threads per grid
-// dimension, so channels past kAbsmaxBlocks go to the grid's second dimension.
-constexpr int64_t kAbsmaxBlocks = 1 << 20;
-
+// V elements of T per load (1: any base and K).
 template <typename T, int V>
 __global__ __launch_bounds__(256) void fp8_absmax_kernel(const T* __restrict__ w, T* __restrict__ amax_out, int64_t N,
                                                          int64_t K) {
   typedef T tv_t __attribute__((ext_vector_type(V)));
   __shared__ float part[4];
-  const int64_t n = (int64_t)blockIdx.y * kAbsmaxBlocks + blockIdx.x;
+  const int64_t n = ldk::tile_index();
   if (n >= N) return;  // uniform
   const T* row = w + n * K;
   float amax = 0.0f;
@@ -110,7 +107,8 @@ __global__ __launch_bounds__(256) void fp8_quantize_kernel(const T* __restrict__
   typedef T tv_t __attribute__((ext_vector_type(V)));
   __shared__ __align__(4) uint8_t tile[kFRows][kFCols + 4];
   const int64_t kt = (K + kFRows - 1) / kFRows;
-  const int64_t k0 = blockIdx.x % kt * kFRows, n0 = blockIdx.x / kt * kFCols;
+  const int64_t t = ldk::tile_index(), k0 = t % kt * kFRows, n0 = t / kt * kFCols;
+  if (n0 >= N) return;  // uniform
   constexpr int LPR = kFRows / V, P = kFCols * LPR / 256;  // lanes per channel, passes
   constexpr int U = P < 8 ? P : 8;                         // loads in flight
   const int tid = threadIdx.x, kk = tid % LPR * V;
@@ -182,7 +180,8 @@ __global__ __launch_bounds__(256) void fp8_dequant_kernel(const uint8_t* __restr
   constexpr int C = 64, E = 16 / sizeof(T);  // tile side, elements per 16-byte store
   __shared__ __align__(16) T tile[C][C + E];
   const int64_t kt = (K + C - 1) / C;
-  const int64_t k0 = blockIdx.x % kt * C, n0 = blockIdx.x / kt * C;
+  const int64_t tl = ldk::tile_index(), k0 = tl % kt * C, n0 = tl / kt * C;
+  if (n0 >= N) return;  // uniform
   const int tid = threadIdx.x, c = tid % 16 * 4, kr = tid / 16 * 4;
   // L == 4: a word that would pass its row's end starts at N - 4 and is shifted
   const int64_t at = min(n0 + c, N - 4);
@@ -974,15 +973,15 @@ inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t - 1) / t
 template <typename T>
 int launch_fp8_quantize(const T* w, uint8_t* wq, T* scale, int64_t N, int64_t K, hipStream_t s) {
   const int64_t tiles = ((N + kFCols - 1) / kFCols) * ((K + kFRows - 1) / kFRows);
-  if (tiles > INT32_MAX || N > INT32_MAX) return ldk::fail(LDK_ERR_UNSUPPORTED, "fp8_quantize: too large");
+  if (!ldk::tiles_fit(tiles) || N > (int64_t)UINT32_MAX - 255) return ldk::fail(LDK_ERR_UNSUPPORTED, "fp8_quantize: too large");
   const bool vec = K % 8 == 0 && ldk::aligned(w, 16);
-  const dim3 rows((unsigned)std::min(N, kAbsmaxBlocks), (unsigned)((N + kAbsmaxBlocks - 1) / kAbsmaxBlocks));
+  const dim3 rows = ldk::tile_grid(N), grid = ldk::tile_grid(tiles);
   (void)hipGetLastError();
   if (vec)
     fp8_absmax_kernel<T, 8><<<rows, 256, 0, s>>>(w, scale, N, K);
   else
     fp8_absmax_kernel<T, 1><<<rows, 256, 0, s>>>(w, scale, N, K);
-  auto tile = [&](auto kernel) { kernel<<<(unsigned)tiles, 256, 0, s>>>(w, scale, wq, N, K); };
+  auto tile = [&](auto kernel) { kernel<<<grid, 256, 0, s>>>(w, scale, wq, N, K); };
   if (vec && N % 4 == 0)
     tile(fp8_quantize_kernel<T, 8, false>);
   else if (vec)
@@ -998,10 +997,10 @@ int launch_fp8_quantize(const T* w, uint8_t* wq, T* scale, int64_t N, int64_t K,
 template <typename T>
 int launch_fp8_dequant(const uint8_t* wq, const T* scale, T* out, int64_t N, int64_t K, hipStream_t s) {
   const int64_t tiles = ((N + 63) / 64) * ((K + 63) / 64);
-  if (tiles > INT32_MAX) return ldk::fail(LDK_ERR_UNSUPPORTED, "fp8_dequant: too large");
+  if (!ldk::tiles_fit(tiles)) return ldk::fail(LDK_ERR_UNSUPPORTED, "fp8_dequant: too large");
   const bool vec = K * (int64_t)sizeof(T) % 16 == 0 && ldk::aligned(out, 16);
   (void)hipGetLastError();
-  auto tile = [&](auto kernel) { kernel<<<(unsigned)tiles, 256, 0, s>>>(wq, scale, out, N, K); };
+  auto tile = [&](auto kernel) { kernel<<<ldk::tile_grid(tiles), 256, 0, s>>>(wq, scale, out, N, K); };
   if (N >= 4 && vec)
     tile(fp8_dequant_kernel<T, 4, true>);
   else if (N >= 4)

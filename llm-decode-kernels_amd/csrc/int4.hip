@@ -239,7 +239,8 @@ __global__ __launch_bounds__(256) void w4a16_dequant_kernel(const uint32_t* __re
                                                             int64_t K, int gshift_rows) {
   __shared__ __align__(16) half8_t tile[kDCols][kDRows];
   const int64_t R = K / 8, rt = (R + kDRows - 1) / kDRows;
-  const int64_t r0 = blockIdx.x % rt * kDRows, n0 = blockIdx.x / rt * kDCols;
+  const int64_t t = ldk::tile_index(), r0 = t % rt * kDRows, n0 = t / rt * kDCols;
+  if (n0 >= N) return;  // uniform
   const int tid = threadIdx.x, c = tid & (kDCols - 1);
   const int64_t nc = min(n0 + c, N - 1);  // columns and rows past the end repeat the last ones
   uint32_t word[4];
@@ -351,9 +352,9 @@ extern "C" int ldk_w4a16_dequant(const int32_t* qweight, const void* scales, con
     return ldk::fail(LDK_ERR_INVALID, "w4a16_dequant: need K %% 8 == 0, group_size a power of two >= 8 dividing K (K=%lld, group_size=%d)", (long long)K, group_size);
   if (!ldk::aligned(out, 16)) return ldk::fail(LDK_ERR_ALIGN, "w4a16_dequant: out must be 16-byte aligned");
   const int64_t tiles = ((N + kDCols - 1) / kDCols) * ((K / 8 + kDRows - 1) / kDRows);
-  if (tiles > INT32_MAX) return ldk::fail(LDK_ERR_UNSUPPORTED, "w4a16_dequant: too large");
+  if (!ldk::tiles_fit(tiles)) return ldk::fail(LDK_ERR_UNSUPPORTED, "w4a16_dequant: too large");
   (void)hipGetLastError();
-  w4a16_dequant_kernel<<<(unsigned)tiles, 256, 0, (hipStream_t)stream>>>(
+  w4a16_dequant_kernel<<<ldk::tile_grid(tiles), 256, 0, (hipStream_t)stream>>>(
       (const uint32_t*)qweight, (const half_t*)scales, (const half_t*)zeros, (half_t*)out, N, K, gsh - 3);
   return ldk::check_launch("w4a16_dequant");
 }

@@ -248,4 +248,14 @@ inline float* splitk_side(void* ws, int64_t words) {
   return reinterpret_cast<float*>(static_cast<char*>(ws) + (((size_t)words * 8 + 255) & ~size_t(255)));
 }
 
+// Grids of one workgroup per tile of a two-dimensional array of any size: a launch holds fewer than
+// 2^32 threads per grid dimension, so tiles past kGridTiles go to the second. The last row of the grid
+// can pass the last tile.
+constexpr int64_t kGridTiles = 1 << 20;
+inline bool tiles_fit(int64_t tiles) { return tiles <= 65535 * kGridTiles; }
+inline dim3 tile_grid(int64_t tiles) {
+  return dim3((unsigned)(tiles < kGridTiles ? tiles : kGridTiles), (unsigned)((tiles + kGridTiles - 1) / kGridTiles));
+}
+__device__ __forceinline__ int64_t tile_index() { return (int64_t)blockIdx.y * kGridTiles + blockIdx.x; }
+
 }  // namespace ldk

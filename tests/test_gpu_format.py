@@ -233,6 +233,47 @@ def test_fp8_quantize_many_channels(N):
     assert np.array_equal(to_np(wq.view(torch.uint8)[:, rows]), owq.view(np.uint8))
 
 
+@pytest.mark.parametrize("N,K", [(1, (1 << 30) + 72), ((1 << 30) + 130, 1)])
+def test_fp8_more_tiles_than_one_grid_dimension(N, K):
+    """One row or one column of more than 2^24 tiles (2^32 threads in all): codes, scales and the
+    values back, in windows at both ends and around the first tile of the grid's second row."""
+    from kernels.fp8 import FP8, dequantize_fp8, quantize_fp8
+    from oracle import fp8 as of
+
+    w = torch.empty(N, K, dtype=torch.float16, device="cuda").normal_(std=0.05)
+    wq, s = quantize_fp8(w)
+    back = dequantize_fp8(wq, s)
+    n = max(N, K)
+    for at in (0, (64 << 20) - 70, (128 << 20) - 70, n - 140):
+        win = slice(at, at + 140)
+        if K == 1:
+            owq, os_ = of.quantize_fp8(w[win].cpu().numpy())
+            got, sc, ref = wq[:, win], s[win], of.dequantize_fp8(owq, os_)
+        else:
+            top = float(w.abs().max())
+            row = np.append(w[:, win].cpu().numpy(), np.float16([[top]]), 1)  # the row's absmax with the window
+            owq, os_ = of.quantize_fp8(row)
+            owq, got, sc = owq[:-1], wq[win], s
+            ref = of.dequantize_fp8(owq, os_)
+        assert np.array_equal(to_np(got.contiguous().view(torch.uint8)), owq) and np.array_equal(bits16(sc), bits16(os_))
+        b = back[win] if K == 1 else back[:, win]
+        assert np.array_equal(bits16(b.contiguous()), bits16(ref))
+
+
+def test_dequantize_more_tiles_than_one_grid_dimension():
+    """One column of more than 2^24 tiles of 16 packed rows."""
+    R, G = (1 << 28) + 16, 1 << 7
+    g = torch.Generator(device="cuda").manual_seed(1)
+    qw = torch.randint(-(2 ** 31), 2 ** 31 - 1, (R, 1), generator=g, device="cuda", dtype=torch.int64).int()
+    s = torch.rand(R * 8 // G, 1, generator=g, device="cuda").half()
+    z = torch.randint(0, 16, (R * 8 // G, 1), generator=g, device="cuda").half()
+    out = dequantize(qw, s, z, G)
+    for r in (0, (1 << 24) - 32, R - 64):  # windows of 64 packed rows, whole groups
+        win, grp = slice(r, r + 64), slice(r * 8 // G, (r + 64) * 8 // G)
+        ref = dequantize_ref(to_np(qw[win]), to_np(s[grp]), to_np(z[grp]), G)
+        assert np.array_equal(bits16(out[:, r * 8:(r + 64) * 8].contiguous()), bits16(ref))
+
+
 @pytest.mark.parametrize("N", [1, 5, 64])
 def test_fp8_dequantize_every_code(N):
     """The conversion instruction against the format's table: every code times scales of both signs,
