@@ -797,9 +797,11 @@ __global__ __launch_bounds__(kPWaves * 64) void prefill_attention_kernel(const h
 // 16-token tile's last position, fp16 numerators, fp32 sums; the softmax scale is applied in the
 // exponent, exp2((s - m) * scale * log2 e), with one fma instead of a product and a difference.
 //
-// What bounds it: about 4 vector instructions per MFMA (exponent, sum, conversion, maximum), which
-// take the wave's issue slots next to the MFMAs' (one MFMA with four fma's between takes 24 cycles
-// on this chip, 16 without), next to 16 KB of loads to LDS per 32 positions of a workgroup. Measured
+// What bounds it: the vector instructions (6.0 per MFMA over the whole launch at 3000 tokens of 12/2
+// heads, 10.9 at 1024 on blocks of 64: exponent, sum, conversion, maximum), which take the wave's issue
+// slots next to the MFMAs' (one MFMA with four fma's between takes 24 cycles on this chip, 16 without),
+// the 16 KB of loads to LDS per 32 positions of a workgroup, and the unequal workgroups: over the
+// launch the vector unit is 32% busy, the matrix cores 17%, no LDS bank conflicts. Measured
 // (both launches, graph replays, us; runs on different boxes): 12/2 heads at 3000 tokens 147-157 ->
 // 67-78, at 6000 463-465 -> 172-180, 1024 after 3000 cached 105 -> 61; 28/4 heads at 1500 106 -> 51;
 // 16/16 at 816 44 -> 29 (of these the first launch 10.7 -> 7.6 and 16.3 -> 8.0). Error against 64 bits,

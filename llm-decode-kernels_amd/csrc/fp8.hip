@@ -63,7 +63,8 @@ __device__ __forceinline__ uint16_t from_f32<uint16_t>(float v) {
 //  3. fp8_scale_kernel: scale[n] = the rounded fp32 scale.
 // Arithmetic as fp8.py:27-29 in float32: scale = max(absmax / 448, 1e-12);
 // wq = e4m3(clamp(w / scale, -448, 448)). One thread per channel, reading its row twice, took
-// 1293 us on 14336 x 4096 fp16; this 54 us a call, of which the first launch is about 20.
+// 1293 us on 14336 x 4096 fp16; this 52-54 us a call, of which the first launch is about 20, at the
+// copy's rate, and the second about 30, bound by its vector instructions (81% busy).
 __device__ __forceinline__ float fp8_scale(float amax) { return fmaxf(amax / 448.0f, 1e-12f); }
 
 // V elements of T per load (1: any base and K).
@@ -168,11 +169,12 @@ __global__ __launch_bounds__(256) void fp8_quantize_kernel(const T* __restrict__
 // product of an e4m3 value and an fp16/bf16 scale is exact in fp32). Tiles of 64 channels x 64 k
 // turned through LDS: a thread decodes 4 channels x 4 k and leaves each channel's 4 values as one
 // LDS write; an output row leaves in 16-byte stores (VS; one value each where the rows are not
-// 16-byte aligned). L: bytes per load (4 at any address, 1 for N < 4). Bound by the vector
-// instructions per value next to memory, so the codes go through v_cvt_pk_f32_fp8, two at a time:
-// decoded in software, with byte loads where the k rows are not 4-byte aligned, 14336 x 4096 fp16 took
-// 34.8 us a call, 14333 x 4096 39.9 and 1533 x 8960 bf16 14.9; this 27.7, 27.9 and 10.4 (one thread
-// per output, each reading a byte of its own line, 236 us and 66 for the first and the last).
+// 16-byte aligned). L: bytes per load (4 at any address, 1 for N < 4). The codes go
+// through v_cvt_pk_f32_fp8, two at a time: decoded in software, which its vector instructions bound,
+// with byte loads where the k rows are not 4-byte aligned, 14336 x 4096 fp16 took 34.8 us a call, 14333
+// x 4096 39.9 and 1533 x 8960 bf16 14.9; this 27.7, 27.9 and 10.4 (one thread per output, each reading
+// a byte of its own line, 236 us and 66 for the first and the last): about the copy's rate, the vector
+// unit 37% busy (83% of the LDS cycles are bank conflicts of the transposing writes).
 template <typename T, int L, bool VS>
 __global__ __launch_bounds__(256) void fp8_dequant_kernel(const uint8_t* __restrict__ wq, const T* __restrict__ scale,
                                                           T* __restrict__ out, int64_t N, int64_t K) {

@@ -111,9 +111,9 @@ __global__ void quantize_rtn_kernel(const T* __restrict__ w, uint32_t* __restric
 // columns: LPG lanes hold a column's group, 8 weights (one packed word) each, and meet for its
 // minimum and maximum through DPP (min and max do not depend on the order). The words are turned
 // through LDS, so a packed row is stored as 256 contiguous bytes. The arithmetic per weight is the
-// kernel above's. Bound by memory and, next to it, the quotient per weight. On 14336 x 4096
-// fp16 (149 MB) the one-thread-per-group kernel took 968 us (each lane walking its own 256-byte
-// run, twice); this 42 us, 3.5 TB/s (51 us with the IEEE division per weight).
+// kernel above's. Bound by the vector instructions, the quotient per weight above all (85% busy). On
+// 14336 x 4096 fp16 (149 MB) the one-thread-per-group kernel took 968 us (each lane walking its own
+// 256-byte run, twice); this 38, 3.9 TB/s (51 us with the IEEE division per weight).
 constexpr int kQCols = 64;
 
 template <int CTRL>
@@ -228,8 +228,9 @@ __global__ __launch_bounds__(256) void quantize_rtn_tile_kernel(const T* __restr
 // rows of 64 columns: it reads whole 256-byte runs of each packed row, and turns the decoded
 // 16-byte pieces through LDS (column c's piece r at slot r ^ (c % 16), so neither side has bank
 // conflicts beyond the 16-byte accesses' own), so every output row is stored as 256 contiguous
-// bytes. Reading one word per lane down a column took 66 us on 14336 x 4096 (149 MB); this
-// 35, 4.3 TB/s.
+// bytes. At the copy's rate on 14336 x 4096 (149 MB): 26 us, 5.8 TB/s, where reading one word per lane
+// down a column took 45; under 1M weights that, without the LDS round, was 0.2-0.5 us faster (512 x 256
+// 2.4 against 2.9 us).
 constexpr int kDRows = 16, kDCols = 64;
 
 __global__ __launch_bounds__(256) void w4a16_dequant_kernel(const uint32_t* __restrict__ qw,

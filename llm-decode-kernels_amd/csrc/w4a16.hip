@@ -37,10 +37,10 @@
 //  - VALU kernel (M <= 8, EXACT): ((1024+q) - (1024+z)) * s in packed fp16 is exactly the
 //    reference's dequantized weight (one RNE rounding, kernels/reference.py:35), then dot2 with
 //    each x row. The path when exact dequantization is requested.
-//  - MFMA kernel (from 3 rows): an int32 word holds 8 consecutive K of one column, which is exactly
-//    one lane's B operand of v_mfma_f32_16x16x32_f16. A lane's 128-bit load feeds four 16x16
-//    tiles; B = (q - z) exactly in fp16, A = x rows permuted to the nibble-pair order, the fp32
-//    tile of one group is scaled by s once.
+//  - MFMA kernel (from 3 rows; two on narrow shapes past 2 MB): an int32 word holds 8 consecutive K
+//    of one column, which is exactly one lane's B operand of v_mfma_f32_16x16x32_f16. A lane's
+//    128-bit load feeds four 16x16 tiles; B = 1024 + q, exact in fp16, A = x rows permuted to the
+//    nibble-pair order. A group's fp32 tile, less (1024 + z) * sum x, is scaled by s once.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>

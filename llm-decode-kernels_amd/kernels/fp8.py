@@ -102,7 +102,9 @@ def _tuning(config: dict | None, M: int, N: int, K: int) -> tuple[int, int, int]
 
 def config_for(M: int, N: int, K: int, config: dict | None = None) -> str:
     """What ldk_w8a16_matmul runs for a shape (and `config`), as 'path,block_n=..,split_k=..'
-    (the library's plan query; no GPU needed). Raises as the call would for a refused config."""
+    (the library's plan query; no GPU needed). Raises as the call would for a refused config. Where
+    the choice is "gemm" for N % 16 != 0, `config={"prefill": "gemm"}` still refuses the shape: the
+    GEMM for such N runs as the library's choice only."""
     st, (bn, sk, fl) = _query(M, N, K, *_tuning(config, M, N, K))
     _lib.check(st, "w8a16_config")
     path = "gemm" if fl & _lib.PATH_GEMM else "mfma" if fl & _lib.PATH_MFMA else "valu"
