@@ -1068,9 +1068,10 @@ static bool w8_uses_gemm(int64_t M, int64_t N, int64_t K, int64_t ldx, const voi
   // split K so often that they still stream from most CUs. Weights from HBM, tiles of 128 columns times
   // 16-row blocks, blocks against GEMM: 36 (1536x14336 M = 33) 18.6 / 33.1, 48 (2048x13312 M = 33) 19.4 /
   // 31.4, 72 (3072x8192 M = 48) 20.8 / 25.4, 80 (2560x13312 M = 64) 30.6 / 32.5; 96 (4096x14336 M = 33)
-  // 35 / 29, (1536x13312 M = 128) 34.4 / 35.9, (2048x13312 M = 96) 35 / 29; 144 (6144x4096 M = 33) 24 / 17.
-  // Rows of 8- and 4-byte alignment slow the blocks down more than the GEMM: N = 1544 at 39 / 65
-  // 0.82 / 1.09 of the GEMM's time, 2056 at 51 / 68 0.95 / 1.29; 1028 at 27 / 36 0.65 / 0.97, 1540 at 39 0.99.
+  // 42.2 / 34.8, (1536x13312 M = 128) 34.4 / 35.9, (2048x13312 M = 96) 39.1 / 32.2; 144 (6144x4096 M = 33)
+  // 24.2 / 17.5.
+  // Rows of 8- and 4-byte alignment slow the blocks down more than the GEMM (times over the GEMM's): N =
+  // 1544 at 39 / 65 0.85 / 1.09, 2056 at 51 / 68 0.95 / 1.29; 1028 at 27 / 36 0.65 / 0.97, 1540 at 39 0.99.
   if (N < 8192) {
     const int64_t blocks = (M + 15) / 16, wide = (N + 127) / 128 * blocks;
     const int64_t first = N % 8 ? 36 : N % 16 ? 60 : N < 2048 ? 104 : 96;  // of the GEMM's
